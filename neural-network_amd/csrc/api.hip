@@ -562,6 +562,23 @@ int nnhip_layernorm_linear_w8a32(nnhip_ctx *ctx, const float *h, int rows,
                          nullptr, 0, y, N, nnhip::kEpiBias, nullptr, &lf);
       return;
     }
+    // tall inputs: one LayerNorm launch writes the digit planes of the
+    // 128 x 256-tile GEMM (every column block of the other GEMM normalises
+    // its rows again; 8192 rows, K = 1024, N = 8192: 875 -> 256 us a call)
+    const bool aligned = ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(gamma) |
+                           reinterpret_cast<uintptr_t>(beta) |
+                           reinterpret_cast<uintptr_t>(ln_out)) & 15) == 0;
+    if (aligned && nnhip::gemm_tall_shape(rows, K, N)) {
+      const int mpad = ctx_scratch(ctx, rows, K, N);
+      nnhip::launch_swizzle_rows(st, codes, N, K, ctx->sw.p, false);
+      nnhip::launch_layernorm(st, h, rows, K, gamma, beta, ln_out, ctx->limbs.p,
+                              mpad, ctx->rexp.p);
+      nnhip::launch_gemm_lds(st, nnhip::kAFromDigits, ctx->limbs.p, mpad,
+                             ctx->rexp.p, nullptr, 0, nullptr, nullptr, nullptr,
+                             0, rows, K, N, ctx->sw.p, scales, bias, nullptr, 0,
+                             y, N, nnhip::kEpiBias);
+      return;
+    }
     ctx_scratch(ctx, 1, K, N);
     nnhip::launch_swizzle_rows(st, codes, N, K, ctx->sw.p, false);
     nnhip::launch_gemm_lds(st, nnhip::kAFromLayerNorm, nullptr, 0, nullptr, h,

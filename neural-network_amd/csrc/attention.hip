@@ -917,7 +917,7 @@ __global__ __launch_bounds__(256) void layernorm_split_kernel(
     v[j] = (v[j] - mean) / sd * gv[j] + bv[j];
     mx = fmaxf(mx, fabsf(v[j]));
   }
-  if (live)
+  if (live && y)
     *reinterpret_cast<float4 *>(y + rr * d + k) = make_float4(v[0], v[1], v[2], v[3]);
   if (!limbs) return;
   mx = wave_max_all(mx);
@@ -1144,6 +1144,7 @@ void launch_layernorm(hipStream_t st, const float *h, int rows, int d,
   NNHIP_REQUIRE(d <= 4096, kErrArg, "layernorm: d must be <= 4096");
   NNHIP_REQUIRE(!limbs || (d % 128 == 0 && rows <= mpad), kErrArg,
                 "layernorm: digit output needs d % 128 == 0");
+  NNHIP_REQUIRE(y || limbs, kErrArg, "layernorm: no output");   // y may be null with digits
   if (g_ln_split && (d == 512 || d == 1024) &&
       ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(y) |
         reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(b)) & 15) == 0) {

@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 namespace nnhip {
 
@@ -1066,6 +1067,244 @@ __global__ __launch_bounds__(kLdsThreads) void gemm_lds_kernel(
   for (int tm = tmb + 1; tm < tme; ++tm) row_tile(tm);
 }
 
+// ---------------------------------------------------------------------------
+// int8 MFMA GEMM over digit planes for tall inputs (prompts): 128 x 256 output
+// tiles, 8 waves of 64 x 64, K walked 64 at a time.  Both operands are stored
+// in the MFMA operand layout, so a stage is 40 blocks of 1 KB (4 row blocks x
+// 3 planes x 2 steps, 8 column blocks x 2 steps) copied straight into LDS
+// with global_load_lds, 5 per wave, and every operand read is one
+// conflict-free ds_read_b128.  Three stage buffers: the copies of stage s + 2
+// are issued behind the barrier that opens stage s, so two stages are in
+// flight and a stage costs one barrier.  A wave's stage is 24 MFMAs over 16
+// LDS reads; the exact int32 sums of each digit plane stay in registers for
+// the whole of K (|sum| < 4096 * 127 * 128 < 2^31 at the largest K), so the
+// totals are those of the other two GEMMs and the outputs bit-identical.
+// Bound: the MFMAs.  A stage is 1776 MFMA cycles a SIMD; it takes 0.9 us with
+// few tiles running and 1.3 us with all CUs busy (the rate a large bf16
+// product reaches on this card, 45% of its peak).  8192 x 8192 at K = 1024:
+// 220 us, 1.9 POP/s of digit products (gemm_lds_kernel 333, gemm_limb_kernel
+// 752); 8192 x 1024 at K = 4096: 90 us, 2.3 POP/s (249).  128 x 256 and not
+// 256 x 128: the digits are three bytes an entry and the codes one, so the
+// wide tile loads 23 bytes a clock and CU instead of 32.  Rest: 5.6 us a
+// launch outside the stages (first loads, the epilogue's 64 outputs a lane).
+// ---------------------------------------------------------------------------
+constexpr int kTallM = 128, kTallN = 256, kTallThreads = 512;
+constexpr int kTallStage = 40 * 1024, kTallBufs = 3;
+constexpr int kTallGroup = 8;   // row tiles that share a column tile in turn
+
+// One 1 KB block into LDS: lane i's 16 bytes at src + voff go to dst + 16 i.
+// An asm statement and not the builtin: behind the builtin the compiler waits
+// for every copy in flight before the next LDS read, whatever buffer it reads
+// (it has no register output; gemm_tall_kernel waits for the copies itself).
+__device__ __forceinline__ void tall_copy(const int8_t *src, uint32_t voff, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :: "s"(dst), "v"(voff), "s"(src) : "memory");
+}
+
+template <int EPI>
+__global__ __launch_bounds__(kTallThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gemm_tall_kernel(
+    const int8_t *__restrict__ limbs, int mpad, const int *__restrict__ rexp,
+    int M, int K, int N, const int8_t *__restrict__ wq,
+    const float *__restrict__ scale, const float *__restrict__ bias,
+    const float *__restrict__ resid, int64_t ldr, float *__restrict__ y,
+    int64_t ldy, int ntm, int ntn, RopeArgs ra) {
+  __shared__ __attribute__((aligned(16))) int8_t sm[kTallBufs][kTallStage];
+  __shared__ __attribute__((aligned(16))) int s_e[kTallM];
+  __shared__ int s_pos[EPI == kEpiRope ? kTallM : 1];
+  // contiguous runs of tiles on each XCD; within a run, groups of kTallGroup
+  // row tiles walk the column tiles together (their digits stay in the L2)
+  const int T = ntm * ntn;
+  const int per = (T + 7) / 8;
+  const int wi = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if (wi >= T) return;
+  const int grp = wi / (kTallGroup * ntn);
+  const int gm = min(kTallGroup, ntm - grp * kTallGroup);
+  const int in = wi - grp * kTallGroup * ntn;
+  const int tm = grp * kTallGroup + in % gm, tn = in / gm;
+  const int m0 = tm * kTallM, n0 = tn * kTallN;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = w & 1, wn = w >> 1;          // the wave's 64 x 64 sub-tile
+  const int nch = K / 128, ns = K / 64;
+  if (tid < kTallM) {
+    s_e[tid] = m0 + tid < M ? rexp[m0 + tid] : 0;
+    if constexpr (EPI == kEpiRope) s_pos[tid] = m0 + tid < M ? rope_row_pos(ra, m0 + tid) : -1;
+  }
+
+  // the wave's pieces of a stage: p < 24 digits (plane, row block, step),
+  // else codes (column block, step); blocks past the operands re-read the
+  // last one (their outputs are not stored)
+  const int8_t *src[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    const int p = w * 5 + i;
+    if (p < 24) {
+      const int rb = min((m0 >> 5) + ((p & 7) >> 1), (mpad >> 5) - 1);
+      src[i] = limbs + (int64_t)(p >> 3) * mpad * K + (int64_t)rb * nch * 4096;
+    } else {
+      const int cb = min((n0 >> 5) + ((p - 24) >> 1), (N >> 5) - 1);
+      src[i] = wq + (int64_t)cb * nch * 4096;
+    }
+    src[i] += (p & 1) * 1024;
+  }
+  const uint32_t voff = lane * 16;
+  const uint32_t dst0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t *)sm[0] + w * 5120;
+  auto issue = [&](int s, int b) {
+#pragma unroll
+    for (int i = 0; i < 5; ++i)
+      tall_copy(src[i] + (int64_t)s * 2048, voff, dst0 + b * kTallStage + i * 1024);
+  };
+  v16i acc[2][2][kLimbs];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int l = 0; l < kLimbs; ++l) acc[i][j][l] = v16i{};
+  issue(0, 0);
+  issue(1, 1);                                // K % 128 == 0: ns >= 2
+  int buf = 0;
+  for (int s = 0; s < ns; ++s) {
+    // this stage's own copies done (the next stage's 5 may be in flight),
+    // then every wave's; behind the barrier all waves are done with the
+    // buffer of stage s - 1, which stage s + 2 takes
+    if (s + 1 < ns) asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + 2 < ns) issue(s + 2, buf == 0 ? 2 : buf - 1);
+    const int8_t *pa = sm[buf] + wm * 4096 + lane * 16;
+    const int8_t *pb = sm[buf] + 24 * 1024 + wn * 4096 + lane * 16;
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      v4i a[kLimbs][2], b[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        b[j] = *reinterpret_cast<const v4i *>(pb + j * 2048 + st * 1024);
+#pragma unroll
+      for (int l = 0; l < kLimbs; ++l)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          a[l][i] = *reinterpret_cast<const v4i *>(pa + l * 8192 + i * 2048 + st * 1024);
+#pragma unroll
+      for (int l = 0; l < kLimbs; ++l)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[i][j][l] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[l][i], b[j], acc[i][j][l], 0, 0, 0);
+    }
+    buf = buf == 2 ? 0 : buf + 1;
+  }
+  // epilogue: lane holds column (lane & 31) of rows (t >> 2) * 8 + (lane >> 5)
+  // * 4 + (t & 3), t < 16, of each 32 x 32 sub-tile.  Column pairs (SwiGLU,
+  // RoPE) sit on adjacent lanes: of rows t and t + 1 the even lane takes the
+  // pair of row t and the odd lane that of row t + 1.
+  // Outputs at 32-bit byte offsets from the tile's first one (the launcher
+  // keeps ldy below 2^23); tiles with all 128 rows store without a guard.
+  char *const yt = EPI == kEpiRope ? nullptr
+                                   : reinterpret_cast<char *>(
+                                         y + (int64_t)m0 * ldy + (EPI == kEpiSwiGLU ? n0 / 2 : n0));
+  const uint32_t ldb = (uint32_t)ldy * 4u;
+  auto tile = [&](auto full_) {
+    constexpr bool full = decltype(full_)::value;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int nc = wn * 64 + j * 32 + (lane & 31), n = n0 + nc;
+      if (n0 + wn * 64 + j * 32 >= N) continue;   // whole 32-column blocks (N % 32 == 0)
+      float sc = scale[n], bi = bias[n];
+      // waited for here, not in each of the guarded stores below (where the
+      // wait would also be for the stores before it)
+      asm volatile("" : "+v"(sc), "+v"(bi));
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r0 = wm * 64 + i * 32 + (lane >> 5) * 4;   // + (t >> 2) * 8 + (t & 3)
+        int4 e4[4];                               // exponents of the lane's rows
+#pragma unroll
+        for (int q = 0; q < 4; ++q) e4[q] = *reinterpret_cast<const int4 *>(s_e + r0 + 8 * q);
+        // dequant_epilogue of the exact total, formed in double (|total| <
+        // 2^53) and rounded to float once, as the conversion of the integer is
+        auto value = [&](int t) {
+          const double tot = fma((double)acc[i][j][0][t], 65536.0,
+                                 fma((double)acc[i][j][1][t], 256.0, (double)acc[i][j][2][t]));
+          const int4 e = e4[t >> 2];
+          const int ex = (t & 3) == 0 ? e.x : (t & 3) == 1 ? e.y : (t & 3) == 2 ? e.z : e.w;
+          return fmaf(ldexpf((float)tot, -ex), sc, bi);
+        };
+        if constexpr (EPI == kEpiSwiGLU || EPI == kEpiRope) {
+          const bool odd = lane & 1;
+          // rows of this lane's eight pairs: t = 2 u + odd
+          const int rp = r0 + (odd ? 1 : 0);
+          auto row = [&](int u) { return rp + (u >> 1) * 8 + ((2 * u) & 3); };
+          // RoPE: the rows' positions, then four rows' cos / sin requested
+          // before use
+          const int ne = n & ~1;
+          const int E = ra.H * ra.D, part = EPI == kEpiRope ? ne / E : 0;
+          const int nn = EPI == kEpiRope ? ne % E : 0;
+          const int h = EPI == kEpiRope ? nn / ra.D : 0, jd = EPI == kEpiRope ? nn % ra.D : 0;
+#pragma unroll
+          for (int u0 = 0; u0 < 8; u0 += 4) {
+            int pos[4];
+            float cs[4], sn[4];
+            if constexpr (EPI == kEpiRope) {
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                pos[u] = s_pos[row(u0 + u)];
+                const int64_t o = (int64_t)max(pos[u], 0) * (ra.D >> 1) + (jd >> 1);
+                cs[u] = ra.cosb[o];
+                sn[u] = ra.sinb[o];
+              }
+#pragma unroll
+              for (int u = 0; u < 4; ++u) asm volatile("" : "+v"(cs[u]), "+v"(sn[u]));
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const float v0 = value(2 * (u0 + u)), v1 = value(2 * (u0 + u) + 1);
+              const float got = __shfl_xor(odd ? v0 : v1, 1, kWave);
+              const float g = odd ? got : v0, up = odd ? v1 : got;
+              const int m = m0 + row(u0 + u);
+              if constexpr (EPI == kEpiSwiGLU) {
+                const float o = swiglu_pair(g, up);
+                if (full || m < M)
+                  *reinterpret_cast<float *>(yt + (uint32_t)((uint32_t)(m - m0) * ldb + (nc >> 1) * 4u)) = o;
+              } else {
+                // as rope_store_pair_at
+#pragma clang fp contract(off)
+                const float q0 = part == 2 ? g : g * cs[u] - up * sn[u];
+                const float q1 = part == 2 ? up : g * sn[u] + up * cs[u];
+                float *base = part == 0 ? ra.qrot + (int64_t)m * E + nn
+                                        : (part == 1 ? ra.kc : ra.vc) + (m / ra.S) * ra.seq_stride +
+                                              ((int64_t)h * ra.cap + pos[u]) * ra.D + jd;
+                if (pos[u] >= 0) *reinterpret_cast<float2 *>(base) = make_float2(q0, q1);
+              }
+            }
+          }
+        } else {
+          const uint32_t o0 = (uint32_t)r0 * ldb + nc * 4u;
+          float rs[16];
+          if constexpr (EPI == kEpiResid) {
+#pragma unroll
+            for (int t = 0; t < 16; ++t)
+              rs[t] = resid[(int64_t)min(m0 + r0 + (t >> 2) * 8 + (t & 3), M - 1) * ldr + n];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) asm volatile("" : "+v"(rs[t]));
+          }
+#pragma unroll
+          for (int t = 0; t < 16; ++t) {
+            const int dr = (t >> 2) * 8 + (t & 3);
+            float o = value(t);
+            if constexpr (EPI == kEpiResid) o = rs[t] + o;
+            if (full || m0 + r0 + dr < M) *reinterpret_cast<float *>(yt + (uint32_t)(o0 + dr * ldb)) = o;
+          }
+        }
+      }
+    }
+  };
+  if (EPI != kEpiRope && m0 + kTallM <= M) tile(std::true_type{});
+  else tile(std::false_type{});
+}
+
 __global__ __launch_bounds__(256) void quantize_w8_kernel(
     const float *__restrict__ w, int K, float max_q, int8_t *__restrict__ q,
     float *__restrict__ scales) {
@@ -1313,6 +1552,47 @@ void launch_act_quant(hipStream_t st, const float *x, int64_t ldx, int rows,
 
 int g_limb_k8 = 512;
 
+// Where the 128 x 256-tile GEMM takes a digit-plane product over from the
+// other two: from 96 tiles on.  A tile takes 8 (K = 512) to 60 us (K = 4096)
+// however few there are, and 256 run at once; the other two GEMMs' time grows
+// with the rows throughout.  Measured, best of the other two against this one:
+// K = 1024, N = 8192: 128 tiles (512 rows) 25.7 / 24.2 us, 256 tiles 45.9 /
+// 28.8; N = 3072: 96 tiles 22.7 / 21.9, 48 tiles 13.4 / 21.4; K = 512, N =
+// 4096: 128 tiles 18.9 / 15.7, 64 tiles 11.3 / 14.0; K = 4096, N = 1024: 128
+// tiles 130 / 75, 64 tiles 68.3 / 67.4, 32 tiles 36.0 / 64.1.
+constexpr int kTallMinTiles = 96;
+bool gemm_tall_shape(int rows, int K, int N) {
+  const int64_t tiles = (int64_t)((rows + kTallM - 1) / kTallM) * ((N + kTallN - 1) / kTallN);
+  return tiles >= kTallMinTiles && K % 128 == 0 && N % 32 == 0;
+}
+static bool gemm_tall_takes(int rows, int K, int N, int64_t ldy, int epi,
+                            const RopeArgs *ra) {
+  return gemm_tall_shape(rows, K, N) && ldy < (1 << 23) && epi != kEpiTotals &&
+         !(epi == kEpiRope && ra && ra->kq);
+}
+
+static void launch_gemm_tall(hipStream_t st, const int8_t *limbs, int mpad,
+                             const int *rexp, int rows, int K, int N,
+                             const int8_t *wq, const float *scale,
+                             const float *bias, const float *resid, int64_t ldr,
+                             float *y, int64_t ldy, int epi, const RopeArgs &ra) {
+  const int ntm = (rows + kTallM - 1) / kTallM, ntn = (N + kTallN - 1) / kTallN;
+  const int per = (ntm * ntn + 7) / 8;
+#define NNHIP_GT(E)                                                           \
+  hipLaunchKernelGGL(gemm_tall_kernel<E>, dim3(8 * per), dim3(kTallThreads), 0, \
+                     st, limbs, mpad, rexp, rows, K, N, wq, scale, bias, resid, \
+                     ldr, y, ldy, ntm, ntn, ra)
+  switch (epi) {
+    case kEpiBias: NNHIP_GT(kEpiBias); break;
+    case kEpiResid: NNHIP_GT(kEpiResid); break;
+    case kEpiSwiGLU: NNHIP_GT(kEpiSwiGLU); break;
+    default: NNHIP_GT(kEpiRope); break;
+  }
+#undef NNHIP_GT
+  NNHIP_CHECK(hipGetLastError());
+}
+
+
 // The int8 KV append in gemm_limb_kernel's epilogue needs each head's pairs
 // within one tile row's 16 (32x32 tiles) column pairs.
 bool gemm_limb_q8_ok(int D) { return rope_q8_head_dim_ok(D) && D <= 32; }
@@ -1331,6 +1611,11 @@ void launch_gemm_limb(hipStream_t st, const int8_t *limbs, int mpad,
   const bool q8 = epi == kEpiRope && rz.kq;
   NNHIP_REQUIRE(!q8 || gemm_limb_q8_ok(rz.D), kErrArg,
                 "gemm_limb: int8 KV append needs a power-of-two head dim <= 32");
+  if (gemm_tall_takes(rows, K, N, ldy, epi, ra)) {
+    launch_gemm_tall(st, limbs, mpad, rexp, rows, K, N, wq, scale, bias, resid,
+                     ldr, y, ldy, epi, rz);
+    return;
+  }
   // 32x64 tiles when they alone give enough workgroups to fill the chip,
   // otherwise 32x32 tiles (twice the workgroups, two resident per CU)
   const int ntm = (rows + kGemmMT - 1) / kGemmMT;
@@ -1415,6 +1700,11 @@ void launch_gemm_lds(hipStream_t st, int mode, const int8_t *limbs, int mpad,
   NNHIP_REQUIRE(!ts || !ts->out || (gemm_lds_tile_width(K) > 0 && epi == kEpiBias),
                 kErrArg, "gemm_lds: tile statistics need K of 512 or 1024 and a bias epilogue");
   const TileStatsArgs tz = ts ? *ts : TileStatsArgs{};
+  if (mode == kAFromDigits && !tz.out && gemm_tall_takes(rows, K, N, ldy, epi, ra)) {
+    launch_gemm_tall(st, limbs, mpad, rexp, rows, K, N, wq, scale, bias, resid,
+                     ldr, y, ldy, epi, rz);
+    return;
+  }
   const int ntn = (int)(gemm_lds_workgroups(rows, K, N) / ntm);
   // digit planes: a workgroup walks as many row tiles as it takes for all
   // workgroups to be resident at once (one per CU), so that the weights are

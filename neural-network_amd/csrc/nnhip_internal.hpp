@@ -399,6 +399,9 @@ void launch_gemv(hipStream_t st, const float *x, int64_t ldx, int rows, int K,
 void launch_act_quant(hipStream_t st, const float *x, int64_t ldx, int rows,
                       int K, int8_t *limbs, int mpad, int *rexp);
 bool gemm_limb_q8_ok(int D);
+// whether a product over digit planes is tall enough for the 128 x 256-tile
+// GEMM (launch_gemm_limb and launch_gemm_lds then run that one)
+bool gemm_tall_shape(int rows, int K, int N);
 void launch_gemm_limb(hipStream_t st, const int8_t *limbs, int mpad,
                       const int *rexp, int rows, int K, int N,
                       const int8_t *wq, const float *scale, const float *bias,

@@ -21,7 +21,7 @@ __device__ __forceinline__ int quad_at(int i, int lane, int d) {
 // LayerNorm of one row (layer.cpp:242-261) held by a wave in quads with
 // their gamma / beta: mean = sum / N, var = sum((x - mean)^2) / N,
 // (x - mean) / sqrt(var + 1e-5) * gamma + beta; the sums are DPP wave
-// reductions.  y gets the normalised row; with limbs its digits for the next
+// reductions.  y (unless null) gets the normalised row; with limbs its digits for the next
 // MFMA GEMM (row exponent from the row's max, as aq_row_finish).
 template <int NQ>
 __device__ __forceinline__ void ln_row_finish(
@@ -55,8 +55,9 @@ __device__ __forceinline__ void ln_row_finish(
     float *w = v[i];
 #pragma unroll
     for (int j = 0; j < 4; ++j) w[j] = (w[j] - mean) / sd * gv[i][j] + bv[i][j];
-    *reinterpret_cast<float4 *>(y + (int64_t)row * d + 256 * i + 4 * lane) =
-        make_float4(w[0], w[1], w[2], w[3]);
+    if (y)
+      *reinterpret_cast<float4 *>(y + (int64_t)row * d + 256 * i + 4 * lane) =
+          make_float4(w[0], w[1], w[2], w[3]);
     mx = fmaxf(mx, fmaxf(fmaxf(fabsf(w[0]), fabsf(w[1])),
                          fmaxf(fabsf(w[2]), fabsf(w[3]))));
   }

@@ -750,3 +750,105 @@ def test_spec_accept_odd_vocab(ctx, V):
     statistics read single columns) or end inside a run of tiles."""
     n, ties = accept_case(ctx, 16, 4, V, 0.7, 0.9, seed=V)
     assert ties <= 1
+
+
+def _linear_rows(ctx, x, codes, sc, b, path, step):
+    """nnhip_linear_w8a32 over x in slices of `step` rows."""
+    dc, ds, db = ctx.array(codes), ctx.array(sc), ctx.array(b)
+    out = []
+    for r in range(0, len(x), step):
+        dx = ctx.array(x[r:r + step])
+        y = ctx.array(shape=(len(x[r:r + step]), len(codes)))
+        nnhip.call("nnhip_linear_w8a32", ctx.h, dx.p, y.shape[0], x.shape[1],
+                   dc.p, ds.p, db.p, len(codes), y.p, path)
+        out.append(y.numpy())
+    return np.concatenate(out)
+
+
+@pytest.mark.parametrize("rows,K,N", [
+    (12 * 128 - 127, 128, 8 * 256),        # 96 tiles, the last with one row
+    (4 * 128, 256, 23 * 256 + 64),         # a last column tile of 64
+    (1000, 384, 3072), (2050, 512, 1536), (200, 1024, 12288),
+    (8 * 128 + 37, 4096, 12 * 256 - 192)])
+def test_tall_gemm_matches_short_slices(ctx, rows, K, N):
+    """The 128 x 256-tile GEMM (from 96 tiles on) forms the same exact digit
+    totals and the same rounding as the GEMMs of short inputs, so its rows
+    are bit for bit those of 64-row slices; against float64 within the digit
+    resolution (2^-22 of a row's maximum per entry)."""
+    rng = np.random.default_rng(rows + K)
+    x = rng.standard_normal((rows, K)).astype(np.float32)
+    x[::7] *= 1e-3
+    x[5] = 0
+    codes = rng.integers(-127, 128, (N, K)).astype(np.int8)
+    sc = (rng.random(N) * 0.01 + 1e-4).astype(np.float32)
+    b = rng.standard_normal(N).astype(np.float32)
+    got = _linear_rows(ctx, x, codes, sc, b, 2, rows)
+    np.testing.assert_array_equal(got, _linear_rows(ctx, x, codes, sc, b, 2, 64))
+    pick = np.r_[0, 5, 7, rows - 1]
+    w = codes.astype(np.float64) * sc[:, None]
+    ex = x[pick].astype(np.float64) @ w.T + b
+    # each entry is off by at most half a digit unit, max|x| 2^-22 (the row
+    # exponent keeps |X| < 2^22, at least 2^21); then one fp32 rounding
+    tol = (np.abs(x[pick]).max(1) * 2.0 ** -21)[:, None] * np.abs(w).sum(1) + \
+        np.abs(ex) * 2.0 ** -23 + np.abs(b) * 2.0 ** -23 + 1e-30
+    assert (np.abs(got[pick] - ex) <= tol).all()
+
+
+def test_tall_layernorm_linear(ctx):
+    """nnhip_layernorm_linear_w8a32 on a tall input (one LayerNorm launch,
+    then the 128 x 256-tile GEMM), with and without ln_out, against float64."""
+    rows, K, N = 1570, 512, 2048
+    rng = np.random.default_rng(3)
+    h = (rng.standard_normal((rows, K)) + 0.2).astype(np.float32)
+    g = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    be = (0.1 * rng.standard_normal(K)).astype(np.float32)
+    codes = rng.integers(-127, 128, (N, K)).astype(np.int8)
+    sc = np.full(N, 0.002, np.float32)
+    b = rng.standard_normal(N).astype(np.float32)
+    a = [ctx.array(v) for v in (h, g, be, codes, sc, b)]
+    ys = []
+    ln, y = ctx.array(shape=(rows, K)), ctx.array(shape=(rows, N))
+    for out in (ln.p, None):
+        nnhip.call("nnhip_layernorm_linear_w8a32", ctx.h, a[0].p, rows, K,
+                   a[1].p, a[2].p, out, a[3].p, a[4].p, a[5].p, N, y.p)
+        ys.append(y.numpy())
+    np.testing.assert_array_equal(ys[0], ys[1])
+    h64 = h.astype(np.float64)
+    hc = h64 - h64.mean(1, keepdims=True)
+    ex = hc / np.sqrt((hc ** 2).mean(1, keepdims=True) + 1e-5) * g + be
+    # LayerNorm: three roundings of values below ~5 and the sums' own errors
+    assert np.abs(ln.numpy() - ex).max() <= 4e-6
+    exy = ex @ (codes.astype(np.float64) * 0.002).T + b
+    # the digits' 2^-22 of the row maximum per entry and ln's 4e-6, random
+    # signs over K entries of |w| <= 0.254
+    assert np.abs(ys[0] - exy).max() <= 5e-6 * 0.254 * np.sqrt(K) * 6
+
+
+@pytest.mark.parametrize("B,S,q8", [(9, 259, False), (3, 500, False), (9, 259, True)])
+def test_tall_forward_matches_sequences_alone(ctx, B, S, q8):
+    """A prompt forward whose projections run on the 128 x 256-tile GEMM
+    (bias, residual, SwiGLU and RoPE epilogues, ragged last tiles) gives each
+    sequence the logits and cache rows it gets alone (GEMMs of short inputs):
+    the products are bit-identical, attention and norms are per sequence."""
+    d, H, F, V, L = 512, 8, 2048, 640, 2
+    m = nnhip.Decoder(ctx, V, d, H, F, L, 512)
+    m.init_normal(5, 0.05)
+    m.quantize()
+    ids = np.random.default_rng(S).integers(0, V, (B, S)).astype(np.int32)
+    many = nnhip.KVCache(m, B, q8)
+    got = m.forward(ids, many)
+    for b in (0, B - 1):
+        one = nnhip.KVCache(m, 1, q8)
+        want = m.forward(ids[b:b + 1], one)
+        np.testing.assert_allclose(got[b], want[0], rtol=0,
+                                   atol=2e-6 * np.abs(want).max())
+        read = (lambda c, i: c.read_q8(1, i, H, 64)) if q8 else \
+            (lambda c, i: c.read(1, i, H, 64))
+        for u, v in zip(read(many, b), read(one, 0)):
+            if u.dtype == np.int8:
+                assert (u != v).mean() <= 1e-4
+            else:
+                np.testing.assert_allclose(u, v, rtol=0, atol=2e-6 * np.abs(v).max())
+        one.free()
+    many.free()
+    m.free()
