@@ -118,47 +118,111 @@ __global__ __launch_bounds__(kBlock) void unary_kernel(
     o[operand_offset(i, dout, dout)] = apply_unary(op, a[operand_offset(i, dout, da)]);
 }
 
-// 2-D matmul on 64 x 64 output tiles: a 16 x 16 thread block, each thread
-// 4 x 4 outputs; K staged through LDS 16 at a time.  Every output adds its
-// products in ascending k, each product and sum rounded on its own.
-constexpr int kMT = 64, kKT = 16;
-__global__ __launch_bounds__(kBlock) void matmul_kernel(
+// 2-D matmul on (THR / 16 * TR) x (16 TC) output tiles, TR x TC outputs a
+// thread; K goes through LDS 32 at a time, the next 32 held in registers
+// meanwhile (two LDS buffers, one barrier per 32).  Every output adds its
+// products in ascending k, each product and sum rounded on its own: 2 VALU
+// instructions a product, so 39 TFLOP/s (at 2.4 GHz) is the card's bound and
+// no split of K is possible.  A wave alone on its SIMD issues one instruction
+// in 8 cycles, so tiles are spread over 8 waves, and the operands are kept
+// with k innermost, so that one 16-byte LDS read serves four k's (rows of 36
+// words: the 16 columns a wave reads fall on different banks).  Operand loads
+// run along whichever dimension of the view is the denser one, so a
+// transposed view reads as coalesced as a row-major one.
+// 1024 x 784 x 1024: 134 -> 51 us, 1024 x 1024 x 100: 165 -> 27, 2048 x 2048
+// x 2048: 480 -> 385 (44.7 TFLOP/s).
+constexpr int kKT = 32;
+// 64 x 64 tiles from 160 of them on, below it 32 x 32 ones (four times the
+// workgroups): 192 tiles 32.2 / 34.3 us (64 / 32), 128 tiles 30.8 / 23.8, 32
+// tiles 56 / 27, 1024 tiles 385 / 555.
+constexpr int kMatmulTiles64 = 160;
+template <int TR, int TC, int THR>
+__global__ __launch_bounds__(THR) void matmul_kernel(
     const float *__restrict__ a, int64_t sa0, int64_t sa1,
     const float *__restrict__ b, int64_t sb0, int64_t sb1,
     float *__restrict__ o, int64_t so0, int64_t so1, int M, int N, int K) {
-  __shared__ float As[kKT][kMT + 1];
-  __shared__ float Bs[kKT][kMT + 1];
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  const int r0 = blockIdx.y * kMT, c0 = blockIdx.x * kMT;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += kKT) {
-    for (int e = threadIdx.x; e < kKT * kMT; e += kBlock) {
-      const int kk = e / kMT, mm = e % kMT;
-      const int r = r0 + mm, c = c0 + mm, k = k0 + kk;
-      As[kk][mm] = (r < M && k < K) ? a[r * sa0 + k * sa1] : 0.0f;
-      Bs[kk][mm] = (c < N && k < K) ? b[k * sb0 + c * sb1] : 0.0f;
+  constexpr int MT = THR / 16 * TR, NT = 16 * TC;
+  constexpr int P = kKT + 4;                  // padded row, 16-byte aligned
+  constexpr int LA = kKT * MT / THR, LB = kKT * NT / THR;   // entries per thread
+  constexpr int G = TR * TC >= 8 ? 1 : 2;     // quads of k read together
+  __shared__ __attribute__((aligned(16))) float As[2][MT][P], Bs[2][NT][P];
+  const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
+  const int r0 = blockIdx.y * MT, c0 = blockIdx.x * NT;
+  // the thread's entries of a tile: (k, m) with k or m along the lanes
+  const bool ak = sa1 < sa0, bk = sb0 < sb1;
+  auto at_k = [&](bool along_k, int i, int w) { const int e = tid + i * THR; return along_k ? e % kKT : e / w; };
+  auto at_m = [&](bool along_k, int i, int w) { const int e = tid + i * THR; return along_k ? e / kKT : e % w; };
+  float ra[LA], rb[LB];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {
+      const int k = k0 + at_k(ak, i, MT), r = r0 + at_m(ak, i, MT);
+      ra[i] = (r < M && k < K) ? a[r * sa0 + k * sa1] : 0.0f;
     }
-    __syncthreads();
-    const int kn = min(kKT, K - k0);
-    for (int kk = 0; kk < kn; ++kk) {
-      float av[4], bv[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = As[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bv[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = acc[i][j] + av[i] * bv[j];
+    for (int i = 0; i < LB; ++i) {
+      const int k = k0 + at_k(bk, i, NT), c = c0 + at_m(bk, i, NT);
+      rb[i] = (c < N && k < K) ? b[k * sb0 + c * sb1] : 0.0f;
     }
+  };
+  float acc[TR][TC] = {};
+  fetch(0);
+  for (int k0 = 0, buf = 0; k0 < K; k0 += kKT, buf ^= 1) {
+    // the buffer was last read two tiles ago, before the previous barrier
+#pragma unroll
+    for (int i = 0; i < LA; ++i) As[buf][at_m(ak, i, MT)][at_k(ak, i, MT)] = ra[i];
+#pragma unroll
+    for (int i = 0; i < LB; ++i) Bs[buf][at_m(bk, i, NT)][at_k(bk, i, NT)] = rb[i];
     __syncthreads();
+    if (k0 + kKT < K) fetch(k0 + kKT);
+    // the operands of 4 G k's at a time, the next ones requested before
+    // these are multiplied (the compiler alone reads each right before its
+    // use: an LDS latency per k where a SIMD holds one wave)
+    float4 av[2][G][TR], bv[2][G][TC];
+    auto read = [&](int g, int kk) {
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+#pragma unroll
+        for (int i = 0; i < TR; ++i)
+          av[g][u][i] = *reinterpret_cast<const float4 *>(&As[buf][ty * TR + i][kk + 4 * u]);
+#pragma unroll
+        for (int j = 0; j < TC; ++j)
+          bv[g][u][j] = *reinterpret_cast<const float4 *>(&Bs[buf][tx + 16 * j][kk + 4 * u]);
+      }
+    };
+    auto step = [&](int g, int k) {           // k of the group
+      const int u = k / 4, x = k % 4;
+#pragma unroll
+      for (int i = 0; i < TR; ++i)
+#pragma unroll
+        for (int j = 0; j < TC; ++j)
+          acc[i][j] = acc[i][j] + reinterpret_cast<const float *>(&av[g][u][i])[x] *
+                                      reinterpret_cast<const float *>(&bv[g][u][j])[x];
+    };
+    read(0, 0);
+    if (k0 + kKT <= K) {
+#pragma unroll
+      for (int kk = 0; kk < kKT; kk += 4 * G) {
+        const int g = (kk / (4 * G)) & 1;
+        if (kk + 4 * G < kKT) read(g ^ 1, kk + 4 * G);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < 4 * G; ++k) step(g, k);
+      }
+    } else {
+      for (int kk = 0; kk < K - k0; kk += 4 * G) {
+        read(0, kk);
+#pragma unroll
+        for (int k = 0; k < 4 * G; ++k)
+          if (kk + k < K - k0) step(0, k);
+      }
+    }
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < TR; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = r0 + ty * 4 + i, c = c0 + tx * 4 + j;
+    for (int j = 0; j < TC; ++j) {
+      const int r = r0 + ty * TR + i, c = c0 + tx + 16 * j;
       if (r < M && c < N) o[r * so0 + c * so1] = acc[i][j];
     }
 }
@@ -421,10 +485,16 @@ void launch_matmul(hipStream_t st, const TensorView &a, const TensorView &b,
   NNHIP_REQUIRE(M < (1 << 30) && N < (1 << 30) && K < (1 << 30), kErrArg,
                 "matmul: extent too large");
   if (M == 0 || N == 0) return;
-  const dim3 grid((unsigned)((N + kMT - 1) / kMT), (unsigned)((M + kMT - 1) / kMT));
-  hipLaunchKernelGGL(matmul_kernel, grid, dim3(kBlock), 0, st, at(a), a.strides[0],
-                     a.strides[1], at(b), b.strides[0], b.strides[1], at_mut(out),
-                     out.strides[0], out.strides[1], (int)M, (int)N, (int)K);
+#define NNHIP_MM(TR, TC, THR)                                                 \
+  hipLaunchKernelGGL((matmul_kernel<TR, TC, THR>),                            \
+                     dim3((unsigned)((N + 16 * TC - 1) / (16 * TC)),          \
+                          (unsigned)((M + THR / 16 * TR - 1) / (THR / 16 * TR))), \
+                     dim3(THR), 0, st, at(a), a.strides[0], a.strides[1],     \
+                     at(b), b.strides[0], b.strides[1], at_mut(out),          \
+                     out.strides[0], out.strides[1], (int)M, (int)N, (int)K)
+  if (((M + 63) / 64) * ((N + 63) / 64) >= kMatmulTiles64) NNHIP_MM(2, 4, 512);
+  else NNHIP_MM(1, 2, 512);
+#undef NNHIP_MM
   NNHIP_CHECK(hipGetLastError());
 }
 

@@ -150,6 +150,33 @@ def test_matmul_matches_oracle_dense(ctx, M, K, N):
     np.testing.assert_array_equal(do2.numpy()[:, 0::2], want)
 
 
+@pytest.mark.parametrize("M,K,N", [
+    # 32 x 32 tiles: remainders of rows, columns and of the 32-wide K steps
+    (33, 1, 31), (1, 31, 97), (32, 32, 32), (95, 67, 65), (31, 36, 513),
+    # 64 x 64 tiles (from 160 on), the same remainders
+    (64 * 13 - 63, 33, 64 * 13 - 1), (64 * 10, 64, 64 * 16), (2, 40, 64 * 160)])
+def test_matmul_tiles_bit_exact(ctx, M, K, N):
+    """Both tile sizes at their edges, row-major and transposed operands,
+    against or_dense (ascending k, separately rounded) bit for bit; the
+    entries around the output stay untouched."""
+    rng = np.random.default_rng(M + K + N)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    b = rng.standard_normal((K, N)).astype(np.float32)
+    want = np.zeros((M, N), np.float32)
+    O.lib().or_dense(O.fptr(a), M, K, N, O.fptr(b), None, None, None,
+                     O.fptr(want))
+    keep = np.full((M + 1, N + 3), 7.0, np.float32)
+    for pa, pb in ((False, False), (True, True)):
+        da, va = strided(ctx, a, (1, 0)) if pa else (None, nnhip.view(dev(ctx, a)))
+        db, vb = strided(ctx, b, (1, 0)) if pb else (None, nnhip.view(dev(ctx, b)))
+        do = ctx.array(keep)
+        nnhip.call("nnhip_matmul_f32", ctx.h, va, vb,
+                   nnhip.view(do, (M, N), (N + 3, 1)))
+        got = do.numpy()
+        np.testing.assert_array_equal(got[:M, :N], want)
+        assert (got[M] == 7).all() and (got[:, N:] == 7).all()
+
+
 def test_matmul_known_answer_and_errors(ctx):
     """TensorTest.MatmulContiguous (tensor_test.cpp:82-94): [[1,2,3],[4,5,6]]
     . [[7,8],[9,10],[11,12]] = [[58,64],[139,154]]; shape errors carry the
