@@ -222,6 +222,27 @@ def test_sum_bit_exact(ctx, axes, keep):
     np.testing.assert_array_equal(do.numpy().reshape(want.shape), want)
 
 
+@pytest.mark.parametrize("shape,axes,perm", [
+    ((1024, 100), (0,), None), ((1024, 100), (0,), (1, 0)),
+    ((3, 5000), (1,), None), ((3, 5000), (1,), (1, 0)), ((70001,), (0,), None),
+    ((513, 16, 7), (1,), None), ((257, 33, 3), (0, 2), (2, 0, 1)),
+    ((2, 3000, 5, 2), (0, 1, 3), None), ((600, 15), (1,), None),
+    ((600, 17), (1,), None), ((1, 4, 1), (1,), None), ((5, 0, 3), (1,), None)])
+def test_sum_tiles_bit_exact(ctx, shape, axes, perm):
+    """Long and short sums of one to hundreds of outputs, the loads along
+    either dimension, merged and separate reduced dims, remainders of the
+    tiles and an empty sum: the ascending-order float32 sum bit for bit."""
+    rng = np.random.default_rng(len(shape) + shape[0])
+    x = rng.standard_normal(shape).astype(np.float32)
+    want = serial_sum(x, axes, False) if x.size else np.zeros((5, 3), np.float32)
+    dx, vx = strided(ctx, x, perm) if perm else (None, nnhip.view(dev(ctx, x)))
+    do = ctx.array(shape=want.shape if want.ndim else (1,))
+    ax = (np.ctypeslib.ctypes.c_int64 * len(axes))(*axes)
+    nnhip.call("nnhip_sum_f32", ctx.h, vx, nnhip.view(do, want.shape), ax,
+               len(axes))
+    np.testing.assert_array_equal(do.numpy().reshape(want.shape), want)
+
+
 def test_reference_tensor_known_answers(ctx):
     """The reference's Tensor KATs through the backend ops: BroadcastingAdd
     (tensor_test.cpp:53-67, [2,3] + [1,3]), ElementwiseSubAndMul (:69-80),
