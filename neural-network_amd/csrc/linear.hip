@@ -1305,6 +1305,216 @@ void gemm_tall_kernel(
   else tile(std::false_type{});
 }
 
+// ---------------------------------------------------------------------------
+// fp32 MFMA GEMM over fp32 rows: y = epi(x . w^T), for fp32 weights with more
+// rows than the GEMV is good for, and for int8 codes of shapes the digit
+// GEMMs do not take (K % 128 or N % 64; the codes become floats in LDS, the
+// scale stays in the epilogue).  Workgroup tile 32 TM x 32 TN, one wave per
+// 32 x 32 sub-tile and K slice (KS of them): K goes through LDS 32 per slice
+// at a time (rows of 36 words, so that the 16-byte operand reads fall on
+// different banks), the next step held in registers meanwhile.
+// Precision: v_mfma_f32_32x32x2_f32 chains 8 products in fp32, four such
+// blocks are added pairwise in fp32, and each 32 products then in double, so
+// the rounding errors of a long K do not pile up (the GEMV's come from up to
+// 16 chained products and 8 tree levels): relative error against float64
+// 7e-8 at any K, the GEMV's 6.4e-8 (K = 64) to 1.1e-7 (K = 4096).
+// Bound: the fp32 MFMAs (128 TFLOP/s for a library product), with the sums'
+// VALU work between them where one wave has its SIMD to itself.  333 x 1544
+// at K = 772: 82 -> 23 us (the GEMV reads the weights once per 8 rows); 2048
+// x 4096 at K = 1024: 942 -> 171 us, 100 TFLOP/s.
+// ---------------------------------------------------------------------------
+typedef float v16f __attribute__((ext_vector_type(16)));
+constexpr int kF32K = 32, kF32P = 36;
+
+template <int TM, int TN, int KS, bool Q8>
+__global__ __launch_bounds__(64 * TM * TN * KS) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_f32_kernel(
+    const float *__restrict__ x, int64_t ldx, int M, int K, int N,
+    const int8_t *__restrict__ wq, const float *__restrict__ wf,
+    const float *__restrict__ scale, const float *__restrict__ bias,
+    const float *__restrict__ resid, int64_t ldr, float *__restrict__ y,
+    int64_t ldy, int epi, int ntm, int ntn, RopeArgs ra) {
+  constexpr int THR = 64 * TM * TN * KS, MT = 32 * TM, NT = 32 * TN;
+  constexpr int LA = 4 / TN, LB = 4 / TM;     // 16-byte pieces per thread
+  constexpr int kA = KS * MT * kF32P, kB = KS * NT * kF32P;
+  constexpr int kStage = 2 * (kA + kB), kRed = KS > 1 ? KS * MT * NT * 2 : 0;
+  __shared__ __attribute__((aligned(16))) float sm[kStage > kRed ? kStage : kRed];
+  // contiguous runs of tiles on each XCD, row tiles of a column tile adjacent
+  const int T = ntm * ntn, per = (T + 7) / 8;
+  const int wi = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if (wi >= T) return;
+  const int tn = wi / ntm, tm = wi % ntm;
+  const int m0 = tm * MT, n0 = tn * NT;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int ks = w / (TM * TN), wm = (w % (TM * TN)) % TM, wn = (w % (TM * TN)) / TM;
+  // piece i of the thread: 4 entries of one row (rows past the operands
+  // re-read the last one, their outputs are not stored; entries past K are 0)
+  constexpr int kStep = KS * kF32K;
+  float4 ra4[LA], rb4[LB];
+  const float *xa[LA];
+  int64_t wo[LB];
+#pragma unroll
+  for (int i = 0; i < LA; ++i) {
+    const int p = tid + i * THR, r = (p >> 3) % MT, s = (p >> 3) / MT;
+    xa[i] = x + (int64_t)min(m0 + r, M - 1) * ldx + s * kF32K + 4 * (p & 7);
+  }
+#pragma unroll
+  for (int i = 0; i < LB; ++i) {
+    const int p = tid + i * THR, r = (p >> 3) % NT, s = (p >> 3) / NT;
+    wo[i] = (int64_t)min(n0 + r, N - 1) * K + s * kF32K + 4 * (p & 7);
+  }
+  auto load_w = [&](int i, int k0) {
+    if constexpr (Q8) {
+      const int c = *reinterpret_cast<const int *>(wq + wo[i] + k0);
+      return make_float4((float)(int8_t)c, (float)(int8_t)(c >> 8), (float)(int8_t)(c >> 16),
+                         (float)(int8_t)(c >> 24));
+    } else {
+      return *reinterpret_cast<const float4 *>(wf + wo[i] + k0);
+    }
+  };
+  auto fetch = [&](int k0) {
+    if (k0 + kStep <= K) {
+#pragma unroll
+      for (int i = 0; i < LA; ++i) ra4[i] = *reinterpret_cast<const float4 *>(xa[i] + k0);
+#pragma unroll
+      for (int i = 0; i < LB; ++i) rb4[i] = load_w(i, k0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < LA; ++i) {
+        const int p = tid + i * THR, k = k0 + (p >> 3) / MT * kF32K + 4 * (p & 7);
+        ra4[i] = k < K ? *reinterpret_cast<const float4 *>(xa[i] + k0) : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+#pragma unroll
+      for (int i = 0; i < LB; ++i) {
+        const int p = tid + i * THR, k = k0 + (p >> 3) / NT * kF32K + 4 * (p & 7);
+        rb4[i] = k < K ? load_w(i, k0) : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+    }
+  };
+  double sum[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) sum[t] = 0.0;
+  // blocks of the current step; half = the first two's sum
+  v16f c[4], half = v16f{};
+  c[2] = c[3] = v16f{};
+  auto put = [&](int buf) {                   // piece p: row p / 8 of [KS][MT]
+    float *const sa = sm + buf * (kA + kB), *const sb = sa + kA;
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {
+      const int p = tid + i * THR;
+      *reinterpret_cast<float4 *>(sa + (p >> 3) * kF32P + 4 * (p & 7)) = ra4[i];
+    }
+#pragma unroll
+    for (int i = 0; i < LB; ++i) {
+      const int p = tid + i * THR;
+      *reinterpret_cast<float4 *>(sb + (p >> 3) * kF32P + 4 * (p & 7)) = rb4[i];
+    }
+  };
+  fetch(0);
+  put(0);
+  if (kStep < K) fetch(kStep);
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += kStep, buf ^= 1) {
+    const float *const sa = sm + buf * (kA + kB), *const sb = sa + kA;
+    // lane (r, h) holds entries 16 h .. + 15 of its row: MFMA step j
+    // contracts entries j and 16 + j
+    const float4 *pa = reinterpret_cast<const float4 *>(
+        sa + (ks * MT + wm * 32 + (lane & 31)) * kF32P + 16 * (lane >> 5));
+    const float4 *pb = reinterpret_cast<const float4 *>(
+        sb + (ks * NT + wn * 32 + (lane & 31)) * kF32P + 16 * (lane >> 5));
+    float4 a[4], b[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) { a[q] = pa[q]; b[q] = pb[q]; }
+    // the next step into the other buffer (its readers passed the barrier
+    // below), the one after it requested
+    if (k0 + kStep < K) {
+      put(buf ^ 1);
+      if (k0 + 2 * kStep < K) fetch(k0 + 2 * kStep);
+    }
+    // four blocks of four MFMAs; between them the previous blocks' sums
+    // (a block's result is read no earlier than one block later)
+    auto block = [&](int q, v16f &c) {
+      c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].x, b[q].x, v16f{}, 0, 0, 0);
+      c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].y, b[q].y, c, 0, 0, 0);
+      c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].z, b[q].z, c, 0, 0, 0);
+      c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].w, b[q].w, c, 0, 0, 0);
+    };
+    block(0, c[0]);
+    c[3] += c[2];                             // of the previous step
+    block(1, c[1]);
+    c[3] += half;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) sum[t] += (double)c[3][t];
+    block(2, c[2]);
+#pragma unroll
+    for (int t = 8; t < 16; ++t) sum[t] += (double)c[3][t];
+    block(3, c[3]);
+    half = c[0] + c[1];
+    __syncthreads();
+  }
+  c[3] += c[2];
+  c[3] += half;
+#pragma unroll
+  for (int t = 0; t < 16; ++t) sum[t] += (double)c[3][t];
+  if constexpr (KS > 1) {
+    // the slices' sums added in slice order: each slice's waves then own
+    // 16 / KS of the sub-tile's row groups
+    double *red = reinterpret_cast<double *>(sm);
+    const int st = wn * TM + wm;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) red[((st * KS + ks) * 16 + t) * 64 + lane] = sum[t];
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      if (t / (16 / KS) != ks) continue;
+      double d = red[(st * KS * 16 + t) * 64 + lane];
+#pragma unroll
+      for (int s = 1; s < KS; ++s) d += red[((st * KS + s) * 16 + t) * 64 + lane];
+      sum[t] = d;
+    }
+  }
+  // epilogue: lane holds column (lane & 31) of rows (t >> 2) * 8 + (lane >> 5)
+  // * 4 + (t & 3); column pairs on adjacent lanes, of rows t and t + 1 the
+  // even lane takes row t's pair and the odd lane row t + 1's
+  const int n = n0 + wn * 32 + (lane & 31), nl = min(n, N - 1);
+  float sc = Q8 ? scale[nl] : 1.f, bi = bias[nl];
+  const int r0 = m0 + wm * 32 + (lane >> 5) * 4;
+  float rs[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t)
+    rs[t] = epi == kEpiResid ? resid[(int64_t)min(r0 + (t >> 2) * 8 + (t & 3), M - 1) * ldr + nl] : 0.f;
+  // waited for here, not in each guarded store below
+  asm volatile("" : "+v"(sc), "+v"(bi));
+#pragma unroll
+  for (int t = 0; t < 16; ++t) asm volatile("" : "+v"(rs[t]));
+  // scale and bias in double: one rounding to float
+  auto value = [&](int t) { return (float)(Q8 ? fma(sum[t], (double)sc, (double)bi) : sum[t] + (double)bi); };
+  if (epi == kEpiSwiGLU || epi == kEpiRope) {
+    const bool odd = lane & 1;
+    const int ne = n & ~1;
+#pragma unroll
+    for (int t = 0; t < 16; t += 2) {
+      if (KS > 1 && t / (16 / KS) != ks) continue;
+      const float v0 = value(t), v1 = value(t + 1);
+      const float got = __shfl_xor(odd ? v0 : v1, 1, kWave);
+      const float g = odd ? got : v0, up = odd ? v1 : got;
+      const int m = r0 + (t >> 2) * 8 + (t & 3) + (odd ? 1 : 0);
+      if (m >= M || ne + 1 >= N) continue;
+      if (epi == kEpiSwiGLU) y[(int64_t)m * ldy + ne / 2] = swiglu_pair(g, up);
+      else rope_store_pair(ra, m, ne, g, up);
+    }
+    return;
+  }
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    if (KS > 1 && t / (16 / KS) != ks) continue;
+    const int m = r0 + (t >> 2) * 8 + (t & 3);
+    const float v = value(t);
+    if (m < M && n < N) y[(int64_t)m * ldy + n] = epi == kEpiResid ? rs[t] + v : v;
+  }
+}
+
 __global__ __launch_bounds__(256) void quantize_w8_kernel(
     const float *__restrict__ w, int K, float max_q, int8_t *__restrict__ q,
     float *__restrict__ scales) {
@@ -1478,6 +1688,43 @@ int g_gemm_wide = 1;
 // 1: int8 GEMVs with K of 256-4096 use 128-bit code loads (gemv16_kernel)
 int g_gemv16 = 1;
 
+// The fp32 MFMA GEMM takes a GEMV over from 16 rows and 90000 outputs on: the
+// GEMV runs at about 20 TFLOP/s, the GEMM costs 7 ns per entry of K and wave
+// whatever the size, so the line does not depend on K.  Measured (GEMV /
+// GEMM): 64 x 2048 at K = 512 11.1 / 7.9 us, 64 x 512 at K = 2048 8.5 / 18.4,
+// 128 x 512 at K = 512 6.7 / 7.8, 128 x 3072 at K = 1024 54 / 18.5.
+constexpr int kF32MinRows = 16;
+constexpr int64_t kF32MinOutputs = 90000;
+static void launch_gemm_f32(hipStream_t st, const float *x, int64_t ldx, int rows,
+                            int K, int N, const int8_t *wq, const float *wf,
+                            const float *scale, const float *bias,
+                            const float *resid, int64_t ldr, float *y,
+                            int64_t ldy, int epi, const RopeArgs &ra) {
+#define NNHIP_GF(TM, TN, KS)                                                  \
+  {                                                                           \
+    const int ntm = (rows + 32 * TM - 1) / (32 * TM), ntn = (N + 32 * TN - 1) / (32 * TN); \
+    const dim3 grid(8 * ((ntm * ntn + 7) / 8)), thr(64 * TM * TN * KS);       \
+    if (wq)                                                                   \
+      hipLaunchKernelGGL((gemm_f32_kernel<TM, TN, KS, true>), grid, thr, 0, st, x, \
+                         ldx, rows, K, N, wq, wf, scale, bias, resid, ldr, y, ldy, \
+                         epi, ntm, ntn, ra);                                  \
+    else                                                                      \
+      hipLaunchKernelGGL((gemm_f32_kernel<TM, TN, KS, false>), grid, thr, 0, st, x, \
+                         ldx, rows, K, N, wq, wf, scale, bias, resid, ldr, y, ldy, \
+                         epi, ntm, ntn, ra);                                  \
+  }
+  // 64 x 64 tiles when there are enough of them, else 32 x 32 ones with K over
+  // 4 or 8 waves (2048 x 4096 at K = 1024, 2048 tiles: 175 us with 64 x 64,
+  // 254 with 32 x 32; 512 x 1024, 128 tiles: 32 / 19; 64 x 1024 at K = 4096,
+  // 16 tiles: 41 us over 4 waves, 34 over 8; K below 256 is too short to split)
+  const int64_t t64 = (int64_t)((rows + 63) / 64) * ((N + 63) / 64);
+  if (t64 >= 448 || K < 256) NNHIP_GF(2, 2, 1)
+  else if (t64 > 64 || K < 512) NNHIP_GF(1, 1, 4)
+  else NNHIP_GF(1, 1, 8)
+#undef NNHIP_GF
+  NNHIP_CHECK(hipGetLastError());
+}
+
 void launch_gemv(hipStream_t st, const float *x, int64_t ldx, int rows, int K,
                  int N, const int8_t *wq, const float *wf, const float *scale,
                  const float *bias, const float *resid, int64_t ldr, float *y,
@@ -1492,6 +1739,11 @@ void launch_gemv(hipStream_t st, const float *x, int64_t ldx, int rows, int K,
   NNHIP_REQUIRE(!(ra && ra->kq), kErrArg,
                 "gemv: no int8 KV append in this epilogue (use rope_kv_q8)");
   const RopeArgs rz = ra ? *ra : RopeArgs{};
+  if (!lz.g && rows >= kF32MinRows && (int64_t)rows * N >= kF32MinOutputs) {
+    launch_gemm_f32(st, x, ldx, rows, K, N, wq, wf, scale, bias, resid, ldr, y,
+                    ldy, epi, rz);
+    return;
+  }
   // 32 or more rows (the draft's down projection): groups of 4 rows, twice
   // the workgroups of 8-row groups with half the work each (measured faster)
   if (rows >= 32 && rows % 4 == 0) {

@@ -852,3 +852,75 @@ def test_tall_forward_matches_sequences_alone(ctx, B, S, q8):
         one.free()
     many.free()
     m.free()
+
+
+@pytest.mark.parametrize("q8", [False, True])
+@pytest.mark.parametrize("rows,K,N", [
+    # 64 x 64 tiles, K below 256: remainders of rows, columns and K steps
+    (1407, 64, 64), (1000, 4, 91), (301, 252, 301),
+    # 32 x 32 tiles over 4 waves, then over 8 (64 tiles or fewer)
+    (333, 260, 1544), (500, 772, 1001), (40, 508, 2251), (97, 1000, 929),
+    (16, 4096, 5625), (352, 4092, 257),
+    # 64 x 64 tiles of a large product
+    (1409, 256, 1409)])
+def test_linear_mfma_f32(ctx, rows, K, N, q8):
+    """The fp32 MFMA GEMM of tall fp32 (and odd-shaped int8) inputs: within
+    the rounding of its sums of float64 (chains of 8 products, two pairwise
+    levels, then double and one rounding: 11 roundings at most, each 2^-24 of
+    the row's sum of |x w|), and no further from it than the GEMV's rows."""
+    rng = np.random.default_rng(rows * 7 + K)
+    x = rng.standard_normal((rows, K)).astype(np.float32)
+    b = rng.standard_normal(N).astype(np.float32)
+    dx, db, y = ctx.array(x), ctx.array(b), ctx.array(shape=(rows, N))
+    few = min(rows, 8)
+    y8 = ctx.array(shape=(few, N))
+    if q8:
+        w8 = rng.integers(-127, 128, (N, K)).astype(np.int8)
+        sc = (rng.random(N) * 0.01 + 1e-4).astype(np.float32)
+        w = w8.astype(np.float64) * sc[:, None]
+        dw, ds = ctx.array(w8), ctx.array(sc)
+        for r, o in ((rows, y), (few, y8)):
+            call("nnhip_linear_w8a32", ctx.h, dx.p, r, K, dw.p, ds.p, db.p, N, o.p, 1)
+    else:
+        wf = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+        w = wf.astype(np.float64)
+        dw = ctx.array(wf)
+        for r, o in ((rows, y), (few, y8)):
+            call("nnhip_linear_f32", ctx.h, dx.p, r, K, dw.p, db.p, N, o.p)
+    got = y.numpy()
+    ex = x.astype(np.float64) @ w.T + b
+    size = np.abs(x).astype(np.float64) @ np.abs(w).T + np.abs(b)
+    assert (np.abs(got - ex) <= 11 * 2.0 ** -24 * size).all()
+    err = np.linalg.norm(got - ex) / np.linalg.norm(ex)
+    gemv = np.linalg.norm(y8.numpy() - ex[:few]) / np.linalg.norm(ex[:few])
+    assert err <= 1.1 * gemv + 2e-9, (err, gemv)
+
+
+def test_linear_mfma_f32_inf_nan(ctx):
+    """Infinities and NaN of one row or column stay in it."""
+    rows, K, N = 400, 300, 300
+    x, w = np.ones((rows, K), np.float32), np.full((N, K), 0.5, np.float32)
+    x[3, 7], x[5, 1], w[9, 2] = np.inf, np.nan, -np.inf
+    b = np.zeros(N, np.float32)
+    a = [ctx.array(v) for v in (x, w, b)]
+    y = ctx.array(shape=(rows, N))
+    call("nnhip_linear_f32", ctx.h, a[0].p, rows, K, a[1].p, a[2].p, N, y.p)
+    with np.errstate(invalid="ignore"):
+        ex = x.astype(np.float64) @ w.T
+    np.testing.assert_array_equal(y.numpy(), ex.astype(np.float32))
+
+
+@pytest.mark.parametrize("B,S", [(3, 130), (6, 67)])
+def test_unquantised_forward_tall(ctx, B, S):
+    """A prompt forward of an fp32 model, its projections (bias, residual,
+    SwiGLU and RoPE epilogues) on the fp32 MFMA GEMM, against the oracle."""
+    V, d, H, F, L = 300, 192, 6, 300, 2
+    p = O.make_params(V, d, H, F, L, 11, std=0.1)
+    m = nnhip.Decoder(ctx, V, d, H, F, L, 256)
+    m.set_params(p)
+    o = O.Model(V, d, H, F, L, 256, p, False)
+    ids = np.random.default_rng(B).integers(0, V, (B, S)).astype(np.int32)
+    got = m.forward(ids)
+    for b in range(B):
+        assert_rows_close(got[b], o.forward(ids[b]), what=f"sequence {b}")
+    m.free()
