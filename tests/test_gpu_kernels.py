@@ -685,6 +685,44 @@ def test_sample_rows_top_k_top_p(ctx, V, T, top_k, top_p):
     assert mism <= 1
 
 
+@pytest.mark.parametrize("V", [2, 1023, 4097, 32768])
+@pytest.mark.parametrize("top_k,top_p", [(3, 1.0), (0, 0.6), (40, 0.95), (2000, 0.999)])
+def test_filter_masked_and_equal_rows(ctx, V, top_k, top_p):
+    """The filter at the edges of its digit levels: rows masked with -inf and
+    with the lowest float (more kept ranks than unmasked entries: zeros in
+    index order), one finite entry, all entries equal, probabilities a few
+    ulps apart (in one bin of the first two levels): the kept set of the
+    rule with an exact sum, entries within 1e-6 of the crossing aside.  A
+    row of NaN returns a token in range."""
+    rng = np.random.default_rng(V + top_k)
+    lg = (rng.standard_normal((7, V)) * 3).astype(np.float32)
+    lg[0, V // 3 + 1:] = -np.inf
+    lg[1, 1:] = np.finfo(np.float32).min
+    lg[2, :] = -np.inf
+    lg[2, V // 2] = 1.0
+    lg[3, :] = 0.25
+    lg[4, :] = 1.0 + 1e-6 * rng.integers(0, 5, V)   # 8 ulps apart: expf keeps the order
+    lg[6, V // 2] = np.nan
+    u = rng.random(7).astype(np.float32)
+    dl, du = ctx.array(lg), ctx.array(u)
+    dt, dp = ctx.array(shape=(7,), dtype=np.int32), ctx.array(shape=(7, V))
+    call("nnhip_sample_rows", ctx.h, dl.p, 7, V, 1.0, top_k, top_p, du.p, dt.p,
+         dp.p)
+    tok, got = dt.numpy(), dp.numpy()
+    assert (tok >= 0).all() and (tok < V).all()
+    for b in range(6):
+        z = lg[b].astype(np.float64)
+        p1 = np.exp(z - z.max())
+        p1 /= p1.sum()
+        ke, cs = exact_kept(p1, top_k, top_p)
+        off = (got[b] > 0) != (ke & (p1 > 1e-44))
+        assert not off.any() or np.all(np.abs(cs[off] - top_p) < 1e-6), b
+        if not off.any():
+            want = np.where(ke, p1, 0)
+            assert row_rel_err(got[b][None], (want / want.sum())[None]) <= 1e-5
+            assert got[b][tok[b]] > 0
+
+
 def accept_case(ctx, B, k, V, T, corr, seed):
     rng = np.random.default_rng(seed)
     tl = (rng.standard_normal((B, k, V)) * 2).astype(np.float32)
