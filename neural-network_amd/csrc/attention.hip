@@ -29,6 +29,7 @@ constexpr int kMaxQ = 8;       // queries per workgroup
 // attn_short_q: launches of fewer (sequence, head) pairs than this take
 // their queries in blocks of g_attn_short_q
 constexpr int kAttnShortUnits = 64;
+constexpr int kPromptQ = 20, kPromptGrid = 160;   // attn_prompt_kernel (prompt_shape)
 constexpr int kMaxD = 64;      // head dim handled by the attention kernel
 
 // Embedding gather (cpu_backend.cpp:1020-1025): ids outside [0, vocab) read
@@ -336,6 +337,28 @@ template <> struct KChunk<true> { uint32_t kc[4][2]; float ks[4]; };
 typedef int attn_v4i __attribute__((ext_vector_type(4)));
 typedef int attn_v16i __attribute__((ext_vector_type(16)));
 struct KChunkMfma { attn_v4i kb[2]; float ks; };
+
+// The output projection's digits of one head's 64 entries of a context row
+// (one per lane of the wave): the exponent of the row's head chunk, then X =
+// rint(v 2^e) in balanced base-256 digits (the act_quant_kernel rule applied
+// per head), at k = h * 64 + dd.
+__device__ __forceinline__ void store_head_digits(
+    float v, int64_t row, int h, int dd, int E, int H,
+    int8_t *__restrict__ hlimbs, int mpad, int *__restrict__ hexp) {
+  const float mx = wave_max_all(fabsf(v));
+  const int e = digit_exponent(mx);
+  const int X = (int)rintf(ldexpf(v, e));
+  const int lo = (int)(int8_t)(X & 0xff);
+  const int t1 = (X - lo) >> 8;
+  const int md = (int)(int8_t)(t1 & 0xff);
+  const int hi = (t1 - md) >> 8;
+  const int64_t o = mfma_operand_offset((int)row, h * kWave + dd, E);
+  const int64_t plane = (int64_t)mpad * E;
+  hlimbs[o] = (int8_t)hi;
+  hlimbs[plane + o] = (int8_t)md;
+  hlimbs[2 * plane + o] = (int8_t)lo;
+  if (dd == 0) hexp[row * H + h] = e;
+}
 
 template <int SQP, int DL, int W, bool Q8>
 __global__ __launch_bounds__(kWave * W, W == 4 ? 2 : 1) void attn_kernel(
@@ -699,25 +722,7 @@ __global__ __launch_bounds__(kWave * W, W == 4 ? 2 : 1) void attn_kernel(
       const float inv = ls > 0.f ? 1.0f / ls : 0.f;
       const float v = as * inv;
       out[(row0 + i) * E + h * D + dd] = v;
-      if (D == kWave && hlimbs) {
-        // the output projection's digits of this head's 64 entries of the
-        // row (one per lane of this wave): the exponent of the row's head
-        // chunk, then X = rint(v 2^e) in balanced base-256 digits (the
-        // act_quant_kernel rule applied per head), at k = h D + dd
-        const float mx = wave_max_all(fabsf(v));
-        const int e = digit_exponent(mx);
-        const int X = (int)rintf(ldexpf(v, e));
-        const int lo = (int)(int8_t)(X & 0xff);
-        const int t1 = (X - lo) >> 8;
-        const int md = (int)(int8_t)(t1 & 0xff);
-        const int hi = (t1 - md) >> 8;
-        const int64_t o = mfma_operand_offset((int)(row0 + i), h * D + dd, E);
-        const int64_t plane = (int64_t)mpad * E;
-        hlimbs[o] = (int8_t)hi;
-        hlimbs[plane + o] = (int8_t)md;
-        hlimbs[2 * plane + o] = (int8_t)lo;
-        if (dd == 0) hexp[(row0 + i) * H + h] = e;
-      }
+      if (D == kWave && hlimbs) store_head_digits(v, row0 + i, h, dd, E, H, hlimbs, mpad, hexp);
     }
     return;
   }
@@ -732,6 +737,380 @@ __global__ __launch_bounds__(kWave * W, W == 4 ? 2 : 1) void attn_kernel(
 #pragma unroll
     for (int rr = 0; rr < KPI; ++rr) s += s_buf[(rr * SQP + i) * D + dd];
     part[(((row0 + i) * H + h) * nsplit + sp) * (D + 2) + 2 + dd] = s;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Prompt attention: 32 queries of one (head, sequence) per workgroup on the
+// fp32 MFMA (prompts; the rule is at prompt_shape).  The W
+// waves of a workgroup take the visible 32-key chunks in turn (chunk w, w +
+// W, ...), each with its own online softmax, and merge in LDS as the merged
+// split-K workgroups do; nothing passes between them before that, so the
+// loop has no barrier.
+//  * Scores, transposed (keys x queries): A = K rows, B = the queries, which
+//    stay in registers; lane (c, hh) then holds query c's scores of the 16
+//    keys 8 i + 4 hh + j (i, j < 4).  A step's two dims are d and d + 4 of
+//    an 8-dim block, so that both operands are 16-byte reads.  K rows reach
+//    LDS (rows of D + 4 words: the 16-byte reads of 8 lanes fall on
+//    different banks) through registers loaded one turn ahead.
+//  * Softmax per lane: its 16 keys, one exchange with the other half.
+//  * PV, transposed (dims x queries): step (i, j) multiplies keys 8 i + j and
+//    8 i + 4 + j, which is what the lanes hold, so the probabilities are the
+//    B operand as they are; A = V rows read straight from the cache (a half
+//    wave reads one row; with more than 32 dims, dims 2 c and 2 c + 1 go to
+//    two accumulators).
+// Precision: score sums are 8-product fp32 chains added pairwise; a chunk's
+// 32 products of PV are chained from zero and added to the running rows.
+// int8 rows of 64 dims take the exact integer scores of attn_kernel's MS
+// path; other int8 rows become (float)code * scale as there.
+// A key after some of the tile's queries has p = 0 for them; a V row of such
+// a chunk that is not finite would still spoil their sums (0 * inf), so a
+// chunk with one is summed key by key over the queries that see it.
+// Bound: the fp32 MFMAs, 4096 cycles a chunk (busy 53% of the time; the rest
+// are the softmax's and the sums' 500 VALU instructions a chunk, of which two
+// waves a SIMD hide about half).  RoPE + attention of 4 x 1000 positions, 16
+// heads of 64 dims on 4 KV heads: 323 us on attn_kernel (8 queries a
+// workgroup on the VALU) -> 118; 16 sequences x 40 positions, 16 heads, after
+// 300 cached ones: 39.9 -> 31.3.
+// ---------------------------------------------------------------------------
+typedef float attn_v16f __attribute__((ext_vector_type(16)));
+constexpr int kPromptTile = 32, kPromptWaves = 4;
+
+template <int DL, bool Q8, bool MS>
+__global__ __launch_bounds__(kWave * kPromptWaves, 2) void attn_prompt_kernel(
+    const float *__restrict__ q, KvSrc kv, int S, int H, int Hkv, int cap,
+    const int32_t *__restrict__ base, int off,
+    const int32_t *__restrict__ active, float qscale, float *__restrict__ out,
+    int8_t *__restrict__ hlimbs, int mpad, int *__restrict__ hexp) {
+  constexpr int D = 8 * DL, DP = D + 4, D4 = D / 4;
+  constexpr int ND = DL > 4 ? 2 : 1;          // 32-dim accumulators of PV
+  constexpr int W = kPromptWaves;
+  static_assert(!MS || (Q8 && DL == 8), "integer scores: int8 rows of 64 dims");
+  // per wave: K rows [key][DP], the probabilities of a chunk summed key by
+  // key [key][query], in the end the wave's rows [query][DP]
+  __shared__ float4 s_k4[W][kPromptTile * (DP > kChunk ? DP : kChunk) / 4];
+  __shared__ float s_ml[W][kPromptTile][2];
+  __shared__ float4 s_sc4[Q8 ? W : 1][2][kChunk / 4];   // K, V row scales
+  // neighbouring workgroups go to different XCDs: each XCD gets a run of
+  // (sequence, head) pairs, so the heads of one KV head share its L2
+  const int U = gridDim.x, x = blockIdx.x;
+  const int unit = (U & 7) == 0 ? (x & 7) * (U >> 3) + (x >> 3) : x;
+  const int b = unit / H, h = unit % H;
+  if (active && !active[b]) return;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int c = lane & 31, hh = lane >> 5;
+  float *sk = reinterpret_cast<float *>(s_k4[wv]);
+  // the last tiles see the most keys: they start first
+  const int q0 = (int)(gridDim.y - 1 - blockIdx.y) * kPromptTile;
+  const int nq = min(kPromptTile, S - q0);
+  const int E = H * D, hk = h / (H / Hkv);
+  const int pos0 = base[b] + off + q0;
+  const int kend = min(pos0 + nq, cap);
+  using KT = typename std::conditional<Q8, int8_t, float>::type;
+  const KT *kb = static_cast<const KT *>(kv.k) + b * kv.seq_stride + (int64_t)hk * cap * D;
+  const KT *vb = static_cast<const KT *>(kv.v) + b * kv.seq_stride + (int64_t)hk * cap * D;
+  const float *ksb = Q8 ? kv.ks + b * kv.sc_stride + (int64_t)hk * cap : nullptr;
+  const float *vsb = Q8 ? kv.vs + b * kv.sc_stride + (int64_t)hk * cap : nullptr;
+  const int64_t row0 = (int64_t)b * S + q0;
+
+  // query c: dims 8 f + 4 hh .. + 3, or its digit planes (attn_kernel's MS)
+  const float *qrow = q + (row0 + min(c, nq - 1)) * E + h * D;
+  float4 qf[MS ? 1 : DL];
+  attn_v4i qa[MS ? kLimbs : 1][2];
+  int eq = 0;
+  if constexpr (MS) {
+    float f[2][16], mx = 0.f;
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 v4 = *reinterpret_cast<const float4 *>(qrow + 32 * s2 + 16 * hh + 4 * i);
+        f[s2][4 * i] = v4.x; f[s2][4 * i + 1] = v4.y;
+        f[s2][4 * i + 2] = v4.z; f[s2][4 * i + 3] = v4.w;
+#pragma unroll
+        for (int y = 0; y < 4; ++y) mx = fmaxf(mx, fabsf(f[s2][4 * i + y]));
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    eq = digit_exponent(mx);
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int3 t = digits4(&f[s2][4 * i], eq);
+        qa[0][s2][i] = t.x; qa[1][s2][i] = t.y; qa[2][s2][i] = t.z;
+      }
+  } else {
+#pragma unroll
+    for (int f = 0; f < DL; ++f)
+      qf[f] = *reinterpret_cast<const float4 *>(qrow + 8 * f + 4 * hh);
+  }
+
+  attn_v16f acc[ND];
+#pragma unroll
+  for (int t = 0; t < ND; ++t) acc[t] = attn_v16f{};
+  float m_run = -INFINITY, l_run = 0.f;
+
+  // a chunk's K rows on the way to LDS (piece lane + 64 i: 4 dims of row
+  // piece / D4), or as the integer scores' operand; rows past the last key
+  // re-read it and are masked
+  float4 kr[Q8 ? 1 : DL];
+  uint32_t kc[Q8 && !MS ? DL : 1];
+  attn_v4i kq[2];
+  float kvs = 0.f;                            // int8: row scales, K hh 0, V hh 1
+  auto load_k = [&](int c0) {
+    if constexpr (MS) {
+      const int8_t *p = reinterpret_cast<const int8_t *>(kb) +
+                        (uint32_t)(min(c0 + c, kend - 1) * D + 16 * hh);
+      kq[0] = *reinterpret_cast<const attn_v4i *>(p);
+      kq[1] = *reinterpret_cast<const attn_v4i *>(p + 32);
+    } else {
+#pragma unroll
+      for (int i = 0; i < DL; ++i) {
+        const int p = lane + kWave * i;
+        const KT *src = kb + (uint32_t)(min(c0 + p / D4, kend - 1) * D + 4 * (p % D4));
+        if constexpr (Q8) kc[i] = *reinterpret_cast<const uint32_t *>(src);
+        else kr[i] = *reinterpret_cast<const float4 *>(src);
+      }
+    }
+    if constexpr (Q8) kvs = (hh ? vsb : ksb)[min(c0 + c, kend - 1)];
+  };
+
+  int c0 = wv * kChunk;
+  if (c0 < kend) load_k(c0);
+  for (; c0 < kend; c0 += W * kChunk) {
+    attn_v4i kq_[2] = {};
+    if constexpr (Q8) {
+      reinterpret_cast<float *>(s_sc4[wv][hh])[c] = kvs;
+      if constexpr (MS) { kq_[0] = kq[0]; kq_[1] = kq[1]; }
+      wave_lds_sync();
+    }
+    const float *s_ks = reinterpret_cast<const float *>(s_sc4[Q8 ? wv : 0][0]);
+    if constexpr (!MS) {
+#pragma unroll
+      for (int i = 0; i < DL; ++i) {
+        const int p = lane + kWave * i;
+        float4 k4;
+        if constexpr (Q8) {
+          const float sc = s_ks[p / D4];
+          k4 = make_float4(code_at(kc[i], 0) * sc, code_at(kc[i], 1) * sc,
+                           code_at(kc[i], 2) * sc, code_at(kc[i], 3) * sc);
+        } else {
+          k4 = kr[i];
+        }
+        *reinterpret_cast<float4 *>(sk + (p / D4) * DP + 4 * (p % D4)) = k4;
+      }
+    }
+    // V rows 8 i + 4 hh + j, wanted after the scores
+    // the offsets below are formed anew each turn (kept opaque): hoisted out
+    // of the loop they would hold 16 and more registers each
+    int r0 = c0 + 4 * hh;
+    asm volatile("" : "+v"(r0));
+    const int vcol = ND == 2 ? 2 * min(c, D / 2 - 1) : min(c, D - 1);
+    float v[ND][16];
+    uint16_t vw[Q8 ? 16 : 1];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = min(r0 + 8 * (i >> 2) + (i & 3), kend - 1);
+      const KT *src = vb + (uint32_t)(row * D + vcol);
+      if constexpr (Q8 && ND == 2) {
+        vw[i] = *reinterpret_cast<const uint16_t *>(src);
+      } else if constexpr (Q8) {
+        vw[i] = (uint8_t)*src;
+      } else if constexpr (ND == 2) {
+        const float2 t = *reinterpret_cast<const float2 *>(src);
+        v[0][i] = t.x; v[ND - 1][i] = t.y;
+      } else {
+        v[0][i] = *src;
+      }
+    }
+    wave_lds_sync();
+    float s[16];
+    if constexpr (MS) {
+      attn_v16i sacc[kLimbs];
+#pragma unroll
+      for (int l = 0; l < kLimbs; ++l) sacc[l] = attn_v16i{};
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+        for (int l = 0; l < kLimbs; ++l)
+          sacc[l] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kq_[s2], qa[l][s2], sacc[l], 0, 0, 0);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 sc = *reinterpret_cast<const float4 *>(s_ks + 8 * g + 4 * hh);
+        const float scs[4] = {sc.x, sc.y, sc.z, sc.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = 4 * g + j;
+          const double tot = fma((double)sacc[0][i], 65536.0,
+                                 fma((double)sacc[1][i], 256.0, (double)sacc[2][i]));
+          s[i] = (float)ldexp(tot, -eq) * scs[j];
+        }
+      }
+    } else {
+      // level l of the pairwise sum waits in part[l]
+      attn_v16f part[4];
+#pragma unroll
+      for (int f = 0; f < DL; ++f) {
+        const float4 k4 = *reinterpret_cast<const float4 *>(sk + c * DP + 8 * f + 4 * hh);
+        attn_v16f t = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.x, qf[f].x, attn_v16f{}, 0, 0, 0);
+        t = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.y, qf[f].y, t, 0, 0, 0);
+        t = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.z, qf[f].z, t, 0, 0, 0);
+        t = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, qf[f].w, t, 0, 0, 0);
+        int l = 0;
+#pragma unroll
+        for (int n = f; n & 1; n >>= 1) t += part[l++];
+        part[l] = t;
+        // the sum is wanted here: left to the end, it would keep all blocks'
+        // accumulators
+        if (f & 1) asm volatile("" : "+v"(part[l]));
+      }
+      // blocks left over (DL not a power of two), smallest level first
+      attn_v16f t;
+      bool first = true;
+#pragma unroll
+      for (int l = 0; l < 4; ++l)
+        if ((DL >> l) & 1) {
+          t = first ? part[l] : part[l] + t;
+          first = false;
+        }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = t[i];
+    }
+    __builtin_amdgcn_sched_barrier(0);        // not earlier: registers
+    if (c0 + W * kChunk < kend) load_k(c0 + W * kChunk);
+    __builtin_amdgcn_sched_barrier(0);
+    // chunks that all queries see whole need no mask
+    const bool edge = c0 + kChunk - 1 > pos0 || c0 + kChunk > kend;
+    if (edge) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int key = r0 + 8 * (i >> 2) + (i & 3);
+        s[i] = key <= pos0 + c && key < kend ? s[i] * qscale : -INFINITY;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] *= qscale;
+    }
+    float cm = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) cm = fmaxf(cm, s[i]);
+    cm = fmaxf(cm, __shfl_xor(cm, 32, kWave));
+    const float mn = fmaxf(m_run, cm);
+    const float ms = (mn == -INFINITY) ? 0.f : mn;
+    const float alpha = __builtin_amdgcn_exp2f(m_run - ms);   // 0 at start
+    m_run = mn;
+    float lt[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        s[4 * g + j] = __builtin_amdgcn_exp2f(s[4 * g + j] - ms);   // 0 if masked
+      lt[g] = (s[4 * g] + s[4 * g + 1]) + (s[4 * g + 2] + s[4 * g + 3]);
+    }
+    l_run = l_run * alpha + ((lt[0] + lt[1]) + (lt[2] + lt[3]));
+    if constexpr (Q8) {
+      const float *s_vs = reinterpret_cast<const float *>(s_sc4[wv][1]);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 sc = *reinterpret_cast<const float4 *>(s_vs + 8 * g + 4 * hh);
+        const float scs[4] = {sc.x, sc.y, sc.z, sc.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[0][4 * g + j] = (float)(int8_t)(vw[4 * g + j] & 0xff) * scs[j];
+          if constexpr (ND == 2) v[1][4 * g + j] = (float)(int8_t)(vw[4 * g + j] >> 8) * scs[j];
+        }
+      }
+    }
+    bool plain = true;
+    if (edge) {
+      float big = 0.f;
+#pragma unroll
+      for (int t = 0; t < ND; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) big += 0.f * v[t][i];
+      plain = !__any(big != 0.f);             // NaN after an infinity or a NaN
+    }
+    if (plain) {
+#pragma unroll
+      for (int t = 0; t < ND; ++t) {
+        // four chains of 8 products, added pairwise
+        attn_v16f half[2];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          attn_v16f o{};
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            o = __builtin_amdgcn_mfma_f32_32x32x2f32(v[t][4 * g + j], s[4 * g + j], o, 0, 0, 0);
+          half[g >> 1] = g & 1 ? half[g >> 1] + o : o;
+          if (g & 1) asm volatile("" : "+v"(half[g >> 1]));
+        }
+        const attn_v16f o = half[0] + half[1];
+        acc[t] = acc[t] * alpha + o;
+      }
+    } else {
+      // probabilities [key][query] over the K rows, no longer needed
+#pragma unroll
+      for (int t = 0; t < ND; ++t) acc[t] *= alpha;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sk[(r0 - c0) * kChunk + c + (8 * (i >> 2) + (i & 3)) * kChunk] = s[i];
+      wave_lds_sync();
+      for (int j = 0; j < kChunk && c0 + j < kend; ++j) {
+        const float p = sk[j * kChunk + c];
+        const bool sees = c0 + j <= pos0 + c;
+        const KT *row = vb + (uint32_t)((c0 + j) * D);
+        const KT *rowh = row + 4 * ND * hh;
+#pragma unroll
+        for (int t = 0; t < ND; ++t)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const int d0 = ND * 8 * (e >> 2);      // dims past D: any value
+            const KT vc = (d0 + 4 * ND < D ? rowh : row)[(d0 < D ? d0 : 0) + ND * (e & 3) + t];
+            const float vd = Q8 ? (float)vc * vsb[c0 + j] : (float)vc;
+            acc[t][e] = sees ? acc[t][e] + p * vd : acc[t][e];
+          }
+      }
+    }
+    wave_lds_sync();                          // this turn's LDS reads are done
+  }
+
+  // the wave's rows [query][dim] into its buffer: lane (c, hh) has dims
+  // 8 g + 4 hh .. + 3, or twice that with two accumulators
+  const float l = l_run + __shfl_xor(l_run, 32, kWave);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int d0 = ND * (8 * g + 4 * hh);
+    if (d0 < D) {
+      float *dst = sk + c * DP + d0;
+      if constexpr (ND == 2) {
+        *reinterpret_cast<float4 *>(dst) = make_float4(
+            acc[0][4 * g], acc[ND - 1][4 * g], acc[0][4 * g + 1], acc[ND - 1][4 * g + 1]);
+        *reinterpret_cast<float4 *>(dst + 4) = make_float4(
+            acc[0][4 * g + 2], acc[ND - 1][4 * g + 2], acc[0][4 * g + 3], acc[ND - 1][4 * g + 3]);
+      } else {
+        *reinterpret_cast<float4 *>(dst) = make_float4(
+            acc[0][4 * g], acc[0][4 * g + 1], acc[0][4 * g + 2], acc[0][4 * g + 3]);
+      }
+    }
+  }
+  if (hh == 0) { s_ml[wv][c][0] = m_run; s_ml[wv][c][1] = l; }
+  __syncthreads();
+  for (int t = threadIdx.x; t < nq * D; t += kWave * W) {
+    const int i = t / D, dd = t % D;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < W; ++u) mx = fmaxf(mx, s_ml[u][i][0]);
+    float ls = 0.f, as = 0.f;
+#pragma unroll
+    for (int u = 0; u < W; ++u) {
+      const float mu = s_ml[u][i][0];
+      const float f = mu == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mu - mx);
+      ls += s_ml[u][i][1] * f;
+      as += reinterpret_cast<const float *>(s_k4[u])[i * DP + dd] * f;
+    }
+    const float inv = ls > 0.f ? 1.0f / ls : 0.f;
+    const float o = as * inv;
+    out[(row0 + i) * E + h * D + dd] = o;
+    if (D == kWave && hlimbs) store_head_digits(o, row0 + i, h, dd, E, H, hlimbs, mpad, hexp);
   }
 }
 
@@ -1030,6 +1409,22 @@ bool attention_merged(int D, int max_keys) {
          max_keys <= kMergedWaves * kMergedChunks * kChunk;
 }
 
+// Launches of the prompt kernel: tiles that are not mostly empty, and enough
+// of them.  16 positions a sequence take as long either way and 20 are faster
+// here (16 x 16 heads after 300 keys: 19.8 / 19.7 us, 27.1 -> 20.3); below
+// 160 workgroups the MFMAs of a few CUs would carry the launch that the
+// split-K kernel spreads over the chip (4 heads x 22 tiles: 23.2 us there,
+// 26.6 here; 8 x 22: 22.3 -> 17.2).  Its loads are 16 bytes wide at every head
+// dim and its offsets in a head's rows 32 bits; what is not aligned for them,
+// or longer, stays with the split-K kernel.
+static bool prompt_shape(const float *q, const KvSrc &kv, int B, int S, int H, int D, int cap) {
+  return S >= kPromptQ &&
+         (int64_t)B * H * ((S + kPromptTile - 1) / kPromptTile) >= kPromptGrid && (int64_t)cap * D < (1 << 29) &&
+         ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kv.k) |
+           reinterpret_cast<uintptr_t>(kv.v)) & 15) == 0 &&
+         (kv.seq_stride & (kv.q8 && D == 64 ? 15 : 3)) == 0;
+}
+
 bool launch_attention(hipStream_t st, const float *q, const KvSrc &kv, int B,
                       int S, int H, int Hkv, int D, int cap,
                       const int32_t *base, int off, const int32_t *active,
@@ -1053,7 +1448,41 @@ bool launch_attention(hipStream_t st, const float *q, const KvSrc &kv, int B,
                           (kv.q8 ? 1.0 : 4.0);
   const int nt = !kv.q8 && (g_kv_stream == 2 ||
                             (g_kv_stream == 1 && kv_bytes > kL2StreamBytes));
-  if (attention_merged(D, max_keys)) {
+  const bool merged = attention_merged(D, max_keys);
+  NNHIP_REQUIRE(!hexp || (limbs && D == kWave && (H * D) % 128 == 0 && B * S <= mpad),
+                kErrArg, "attention: head digits need D == 64, H*D % 128 == 0");
+  if (prompt_shape(q, kv, B, S, H, D, cap)) {
+    const dim3 grid(B * H, (S + kPromptTile - 1) / kPromptTile);
+    int8_t *hl = merged && hexp ? limbs : nullptr;
+#define NNHIP_ATTN_MS(DL, Q8, MS)                                             \
+  hipLaunchKernelGGL((attn_prompt_kernel<DL, Q8, MS>), grid,                  \
+                     dim3(kWave * kPromptWaves), 0, st, q, kv, S, H, Hkv, cap, \
+                     base, off, active, qscale, out, hl, mpad, hexp)
+#define NNHIP_ATTN(DL)                                                        \
+  if (kv.q8) NNHIP_ATTN_MS(DL, true, false); else NNHIP_ATTN_MS(DL, false, false)
+    switch (D / 8) {
+      case 1: { NNHIP_ATTN(1); } break;
+      case 2: { NNHIP_ATTN(2); } break;
+      case 3: { NNHIP_ATTN(3); } break;
+      case 4: { NNHIP_ATTN(4); } break;
+      case 5: { NNHIP_ATTN(5); } break;
+      case 6: { NNHIP_ATTN(6); } break;
+      case 7: { NNHIP_ATTN(7); } break;
+      default:
+        // the integer scores where attn_kernel has them; its split launches
+        // form fp32 scores, whose error is the smaller over long contexts
+        if (kv.q8 && merged) NNHIP_ATTN_MS(8, true, true);
+        else { NNHIP_ATTN(8); }
+        break;
+    }
+#undef NNHIP_ATTN
+#undef NNHIP_ATTN_MS
+    NNHIP_CHECK(hipGetLastError());
+    if (merged || !limbs) return false;
+    launch_act_quant(st, out, H * D, B * S, H * D, limbs, mpad, rexp);
+    return true;
+  }
+  if (merged) {
     // one workgroup per (head, sequence, query block); its waves are the key
     // splits, merged in LDS, and the context rows are written directly, with
     // hexp also their digits per head (exponent per row and head).  A launch
@@ -1066,8 +1495,6 @@ bool launch_attention(hipStream_t st, const float *q, const KvSrc &kv, int B,
                          B * H < kAttnShortUnits;
     const int nqb = short_q ? (S + qblk - 1) / qblk : nqb_all;
     const int sq = short_q ? qblk : sq_all;
-    NNHIP_REQUIRE(!hexp || (limbs && D == kWave && (H * D) % 128 == 0 && B * S <= mpad),
-                  kErrArg, "attention: head digits need D == 64, H*D % 128 == 0");
     int8_t *hl = hexp ? limbs : nullptr;
     int kps = (max_keys + kMergedWaves - 1) / kMergedWaves;
     kps = (kps + kChunk - 1) / kChunk * kChunk;

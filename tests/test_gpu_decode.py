@@ -185,6 +185,23 @@ def test_forward_head_digits_vs_oracle(ctx, B, S):
     gm.free()
 
 
+def test_forward_prompt_head_digits(ctx):
+    """The same digits written by the prompt attention (10 x 25 rows of 16
+    heads: 160 tiles)."""
+    om, gm, _ = build(ctx, dict(vocab=512, d=1024, H=16, F=512, L=1), 12, True, std=0.03)
+    ids = np.random.default_rng(25).integers(0, 512, (10, 25)).astype(np.int32)
+    got = gm.forward(ids)
+    ctx.set_option("o_head_digits", 0)
+    try:
+        per_row = gm.forward(ids)
+    finally:
+        ctx.set_option("o_head_digits", 1)
+    for b in range(10):
+        assert_rows_close(got[b], om.forward(ids[b]), 1e-4, f"forward b={b}")
+        assert_rows_close(got[b], per_row[b], 1e-5, f"per-row digits b={b}")
+    gm.free()
+
+
 @pytest.mark.parametrize("B,S", [(1, 5), (32, 1), (32, 6)])
 def test_fused_rope_append_bit_exact(ctx, B, S):
     """The q/k/v epilogue's RoPE and KV append (tensor.cpp:1141-1173,

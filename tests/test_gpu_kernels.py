@@ -427,6 +427,70 @@ def test_attention_short_launch_query_blocks(ctx, qblk, q8):
         ctx.set_option("attn_short_q", 1)
 
 
+# prompts: tiles of 32 positions and chunks of 32 keys dealt to 4 waves:
+# remainders of both, a chunk per wave and more, ragged pasts (up to `past`),
+# every head dim, grouped heads, pair counts that are a multiple of 8 and not;
+# each with the 160 tiles of all pairs that the kernel starts at
+PROMPT_CASES = [(10, 20, 16, 16, 64, 0), (5, 31, 32, 32, 64, 3), (3, 33, 32, 8, 64, 97),
+                (3, 130, 12, 3, 64, 500), (2, 257, 10, 5, 32, 900), (14, 64, 6, 3, 40, 64),
+                (21, 45, 4, 2, 8, 19), (9, 70, 6, 3, 16, 5), (10, 40, 8, 4, 24, 33),
+                (14, 63, 6, 2, 48, 2), (8, 129, 4, 4, 56, 1000)]
+
+
+@pytest.mark.parametrize("q8", [False, True])
+@pytest.mark.parametrize("B,S,H,Hkv,D,past", PROMPT_CASES)
+def test_attention_prompt(ctx, B, S, H, Hkv, D, past, q8):
+    """Prompt launches against the oracle, the caches' unused rows NaN, and
+    one V value infinite at a key that only the later positions see.  Bound:
+    a log2 score here is at most about 12 (unit normal q, k of 64 dims, sum
+    |q k| / 8 * 1.44), formed with about 12 roundings of 2^-24 on each side:
+    9e-6, so 6e-6 of a probability, twice."""
+    rng = np.random.default_rng(S * 100 + D + q8)
+    pos0 = rng.integers(0, past + 1, B).astype(np.int32)
+    pos0[-1] = past
+    cap = int(pos0.max()) + S + 5
+    late = S - 3                       # the new position of the infinite value
+    q = rng.standard_normal((B * S, H * D)).astype(np.float32)
+    dq, dp = ctx.array(q), ctx.array(pos0)
+    do = ctx.array(shape=(B * S, H * D))
+    if q8:
+        k = rng.integers(-127, 128, (B, Hkv, cap, D)).astype(np.int8)
+        v = rng.integers(-127, 128, (B, Hkv, cap, D)).astype(np.int8)
+        v[v == 0] = 1                  # a code times an infinite scale is infinite
+        ks, vs = ((rng.random((B, Hkv, cap)) * 0.01 + 0.005).astype(np.float32)
+                  for _ in range(2))
+        for b in range(B):
+            ks[b, :, pos0[b] + S:] = vs[b, :, pos0[b] + S:] = np.nan
+        vs[0, 0, pos0[0] + late] = np.inf
+        dk, dks, dv, dvs = (ctx.array(a) for a in (k, ks, v, vs))
+        call("nnhip_attention_kq_q8", ctx.h, dq.p, dk.p, dks.p, dv.p, dvs.p, cap,
+             dp.p, B, S, H, Hkv, D, do.p)
+        k = k.astype(np.float32) * ks[..., None]
+        v = v.astype(np.float32) * vs[..., None]
+    else:
+        k = rng.standard_normal((B, Hkv, cap, D)).astype(np.float32)
+        v = rng.standard_normal((B, Hkv, cap, D)).astype(np.float32)
+        for b in range(B):
+            k[b, :, pos0[b] + S:] = v[b, :, pos0[b] + S:] = np.nan
+        v[0, 0, pos0[0] + late, D // 2] = np.inf
+        dk, dv = ctx.array(k), ctx.array(v)
+        call("nnhip_attention_kq", ctx.h, dq.p, dk.p, dv.p, cap, dp.p, B, S, H, Hkv,
+             D, do.p)
+    got = do.numpy().reshape(B, S, H, D)
+    for b in range(B):
+        St = int(pos0[b]) + S
+        kb, vb = (np.ascontiguousarray(a[b, :, :St]) for a in (k, v))
+        qb = np.ascontiguousarray(q[b * S:(b + 1) * S].reshape(S, H, D).transpose(1, 0, 2))
+        out = np.zeros((S, H, D), np.float32)
+        O.lib().or_attention(O.fptr(qb), O.fptr(kb), O.fptr(vb), H, Hkv, S, St, D, 1,
+                             O.fptr(out))
+        fin = np.isfinite(out)
+        assert fin[:late].all() and (b or not fin[late:].all())
+        np.testing.assert_array_equal(np.isfinite(got[b]), fin)
+        assert_rows_close(np.where(fin, got[b], 0).reshape(S, H * D),
+                          np.where(fin, out, 0).reshape(S, H * D), 1.2e-5, f"seq {b}")
+
+
 # grouped-query attention (MultiHeadAttention's num_kv_heads, layer.cpp:
 # 862-864: query head h reads kv head h / (H / H_kv)): the shapes of
 # gqa_test.cpp:115-211 (4 heads on 2 kv heads, B = 2 x 3 queries, and one
@@ -862,12 +926,16 @@ def test_tall_layernorm_linear(ctx):
     assert np.abs(ys[0] - exy).max() <= 5e-6 * 0.254 * np.sqrt(K) * 6
 
 
-@pytest.mark.parametrize("B,S,q8", [(9, 259, False), (3, 500, False), (9, 259, True)])
-def test_tall_forward_matches_sequences_alone(ctx, B, S, q8):
+@pytest.mark.parametrize("B,S,q8", [(9, 300, False), (4, 293, False), (9, 300, True)])
+def test_tall_forward_matches_short_batches(ctx, B, S, q8):
     """A prompt forward whose projections run on the 128 x 256-tile GEMM
-    (bias, residual, SwiGLU and RoPE epilogues, ragged last tiles) gives each
-    sequence the logits and cache rows it gets alone (GEMMs of short inputs):
-    the products are bit-identical, attention and norms are per sequence."""
+    (bias, residual, SwiGLU and RoPE epilogues, ragged last tiles) gives its
+    first and last sequence the logits and cache rows they get as a batch of
+    two (GEMMs of short inputs): the products are bit-identical, attention
+    and norms are per sequence.  Two sequences of 10 position tiles are what
+    the attention's MFMA kernel starts at, so both sides run it: a sequence
+    alone would run the split-K kernel, whose other rounding (1.4e-7 of a row
+    each, from float64) flips codes of an int8 cache."""
     d, H, F, V, L = 512, 8, 2048, 640, 2
     m = nnhip.Decoder(ctx, V, d, H, F, L, 512)
     m.init_normal(5, 0.05)
@@ -875,19 +943,19 @@ def test_tall_forward_matches_sequences_alone(ctx, B, S, q8):
     ids = np.random.default_rng(S).integers(0, V, (B, S)).astype(np.int32)
     many = nnhip.KVCache(m, B, q8)
     got = m.forward(ids, many)
-    for b in (0, B - 1):
-        one = nnhip.KVCache(m, 1, q8)
-        want = m.forward(ids[b:b + 1], one)
-        np.testing.assert_allclose(got[b], want[0], rtol=0,
-                                   atol=2e-6 * np.abs(want).max())
+    two = nnhip.KVCache(m, 2, q8)
+    want = m.forward(ids[[0, B - 1]], two)
+    for i, b in enumerate((0, B - 1)):
+        np.testing.assert_allclose(got[b], want[i], rtol=0,
+                                   atol=2e-6 * np.abs(want[i]).max())
         read = (lambda c, i: c.read_q8(1, i, H, 64)) if q8 else \
             (lambda c, i: c.read(1, i, H, 64))
-        for u, v in zip(read(many, b), read(one, 0)):
+        for u, v in zip(read(many, b), read(two, i)):
             if u.dtype == np.int8:
                 assert (u != v).mean() <= 1e-4
             else:
                 np.testing.assert_allclose(u, v, rtol=0, atol=2e-6 * np.abs(v).max())
-        one.free()
+    two.free()
     many.free()
     m.free()
 
