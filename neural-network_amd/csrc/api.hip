@@ -749,15 +749,17 @@ int nnhip_attention_kq_q8(nnhip_ctx *ctx, const float *q, const int8_t *kcodes,
     hipStream_t st = ctx->c.stream;
     const int max_keys = cap;
     const int64_t pe = nnhip::attention_partial_elems(B, S, H, D, max_keys);
-    nnhip::DevBuf<float> part(pe > 0 ? pe : 1);
+    if ((size_t)std::max<int64_t>(pe, 1) > ctx->part.n) {
+      NNHIP_CHECK(hipStreamSynchronize(st));   // earlier calls may read it
+      ctx->part.ensure((size_t)std::max<int64_t>(pe, 1));
+    }
     nnhip::KvSrc kv;
     kv.q8 = true;
     kv.k = kcodes; kv.v = vcodes; kv.ks = kscales; kv.vs = vscales;
     kv.seq_stride = (int64_t)Hkv * cap * D;
     kv.sc_stride = (int64_t)Hkv * cap;
     nnhip::launch_attention(st, q, kv, B, S, H, Hkv, D, cap, pos0, 0, nullptr,
-                            max_keys, part.p, pe, out);
-    NNHIP_CHECK(hipStreamSynchronize(st));
+                            max_keys, ctx->part.p, pe, out);
   });
 }
 
