@@ -523,17 +523,19 @@ int nnhip_linear_w8a32(nnhip_ctx *ctx, const float *x, int rows, int K,
       NNHIP_REQUIRE(nnhip::gemm_lds_supports(rows, K, N), nnhip::kErrArg,
                     "LDS GEMM needs K in {128, 256, 512, 1024} and N % 32 == 0");
       const int mpad = ctx_scratch(ctx, rows, K, N);
-      nnhip::launch_swizzle_rows(st, codes, N, K, ctx->sw.p, false);
       if (path == 4)
-        nnhip::launch_act_quant(st, x, K, rows, K, ctx->limbs.p, mpad, ctx->rexp.p);
+        nnhip::launch_gemm_operands(st, x, rows, K, ctx->limbs.p, mpad, ctx->rexp.p,
+                                    codes, N, ctx->sw.p);
+      else
+        nnhip::launch_swizzle_rows(st, codes, N, K, ctx->sw.p, false);
       nnhip::launch_gemm_lds(st, path == 4 ? nnhip::kAFromDigits : nnhip::kAFromRows,
                              ctx->limbs.p, mpad, ctx->rexp.p, x, K, nullptr,
                              nullptr, nullptr, 0, rows, K, N, ctx->sw.p, scales,
                              bias, nullptr, 0, y, N, nnhip::kEpiBias);
     } else if (mfma) {
       const int mpad = ctx_scratch(ctx, rows, K, N);
-      nnhip::launch_swizzle_rows(st, codes, N, K, ctx->sw.p, false);
-      nnhip::launch_act_quant(st, x, K, rows, K, ctx->limbs.p, mpad, ctx->rexp.p);
+      nnhip::launch_gemm_operands(st, x, rows, K, ctx->limbs.p, mpad, ctx->rexp.p,
+                                  codes, N, ctx->sw.p);
       nnhip::launch_gemm_limb(st, ctx->limbs.p, mpad, ctx->rexp.p, rows, K, N,
                               ctx->sw.p, scales, bias, nullptr, 0, y, N,
                               nnhip::kEpiBias);

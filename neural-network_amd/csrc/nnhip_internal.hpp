@@ -398,6 +398,10 @@ void launch_gemv(hipStream_t st, const float *x, int64_t ldx, int rows, int K,
                  const GemvLn *ln = nullptr);
 void launch_act_quant(hipStream_t st, const float *x, int64_t ldx, int rows,
                       int K, int8_t *limbs, int mpad, int *rexp);
+// launch_act_quant of x [rows][K] and launch_swizzle_rows of codes [N][K]
+void launch_gemm_operands(hipStream_t st, const float *x, int rows, int K,
+                          int8_t *limbs, int mpad, int *rexp,
+                          const int8_t *codes, int N, int8_t *sw);
 bool gemm_limb_q8_ok(int D);
 // whether a product over digit planes is tall enough for the 128 x 256-tile
 // GEMM (launch_gemm_limb and launch_gemm_lds then run that one)

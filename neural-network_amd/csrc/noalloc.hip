@@ -101,15 +101,17 @@ int nnhip_linear_w8a32_noalloc(nnhip_ctx *ctx, const float *x, int rows,
     int8_t *sw = static_cast<int8_t *>(base);
     int8_t *limbs = sw + sw_bytes;
     int *rexp = reinterpret_cast<int *>(limbs + limb_bytes);
-    nnhip::launch_swizzle_rows(st, codes, N, K, sw, false);
     if (lds) {
-      if (path == 4) nnhip::launch_act_quant(st, x, K, rows, K, limbs, mpad, rexp);
+      if (path == 4)
+        nnhip::launch_gemm_operands(st, x, rows, K, limbs, mpad, rexp, codes, N, sw);
+      else
+        nnhip::launch_swizzle_rows(st, codes, N, K, sw, false);
       nnhip::launch_gemm_lds(st, path == 4 ? nnhip::kAFromDigits : nnhip::kAFromRows,
                              limbs, mpad, rexp, x, K, nullptr, nullptr, nullptr,
                              0, rows, K, N, sw, scales, bias, nullptr, 0, y, N,
                              nnhip::kEpiBias);
     } else {
-      nnhip::launch_act_quant(st, x, K, rows, K, limbs, mpad, rexp);
+      nnhip::launch_gemm_operands(st, x, rows, K, limbs, mpad, rexp, codes, N, sw);
       nnhip::launch_gemm_limb(st, limbs, mpad, rexp, rows, K, N, sw, scales,
                               bias, nullptr, 0, y, N, nnhip::kEpiBias);
     }
