@@ -767,7 +767,7 @@ __global__ __launch_bounds__(kWave * W, W == 4 ? 2 : 1) void attn_kernel(
 // a chunk that is not finite would still spoil their sums (0 * inf), so a
 // chunk with one is summed key by key over the queries that see it.
 // Bound: the fp32 MFMAs, 4096 cycles a chunk (busy 53% of the time; the rest
-// are the softmax's and the sums' 500 VALU instructions a chunk, of which two
+// are the softmax's and the sums' 580 VALU instructions a chunk, of which two
 // waves a SIMD hide about half).  RoPE + attention of 4 x 1000 positions, 16
 // heads of 64 dims on 4 KV heads: 323 us on attn_kernel (8 queries a
 // workgroup on the VALU) -> 118; 16 sequences x 40 positions, 16 heads, after
