@@ -243,8 +243,7 @@ constexpr int kSumBuf = 10240;                // OT * (RC + 4) at most (OT = 512
 
 struct SumDims {
   int rd;                                     // collapsed reduced dims
-  int32_t rshape[kMaxRank];
-  int64_t rstride[kMaxRank];
+  int64_t rshape[kMaxRank], rstride[kMaxRank];
   int kd;                                     // kept dims, row-major
   int64_t kshape[kMaxRank], kin[kMaxRank], kout[kMaxRank];
 };
@@ -605,14 +604,12 @@ void launch_sum(hipStream_t st, const TensorView &in, const TensorView &out,
     if ((mask >> i) & 1u) {
       if (keep) ++od;
       if (in.shape[i] == 1) continue;
-      NNHIP_REQUIRE(in.shape[i] <= 0x7fffffff, kErrArg, "sum: extent too large");
       const int l = d.rd - 1;
-      if (l >= 0 && d.rstride[l] == in.shape[i] * in.strides[i] &&
-          (int64_t)d.rshape[l] * in.shape[i] <= 0x7fffffff) {
-        d.rshape[l] *= (int32_t)in.shape[i];
+      if (l >= 0 && d.rstride[l] == in.shape[i] * in.strides[i]) {
+        d.rshape[l] *= in.shape[i];
         d.rstride[l] = in.strides[i];
       } else {
-        d.rshape[d.rd] = (int32_t)in.shape[i];
+        d.rshape[d.rd] = in.shape[i];
         d.rstride[d.rd++] = in.strides[i];
       }
       continue;

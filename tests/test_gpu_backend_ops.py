@@ -243,6 +243,22 @@ def test_sum_tiles_bit_exact(ctx, shape, axes, perm):
     np.testing.assert_array_equal(do.numpy().reshape(want.shape), want)
 
 
+@pytest.mark.parametrize("shape,axes,strides", [
+    ((2 ** 31 + 9, 0), (0, 1), (0, 1)), ((0, 2 ** 31, 3), (0, 1), (0, 0, 1)),
+    ((70000, 70000, 0), (0, 1, 2), (70000, 1, 1))])
+def test_sum_extents_beyond_32_bits(ctx, shape, axes, strides):
+    """Summed extents past 2^31 - 1, alone and merged, are taken (here with an
+    empty one beside them, so that the sums are 0 and quick)."""
+    kept = [n for d, n in enumerate(shape) if d not in axes]
+    do = ctx.array(np.full(3, 7, np.float32))
+    ax = (np.ctypeslib.ctypes.c_int64 * len(axes))(*axes)
+    nnhip.call("nnhip_sum_f32", ctx.h,
+               nnhip.view(dev(ctx, np.ones(4)), shape, strides),
+               nnhip.view(do, kept), ax, len(axes))
+    n = int(np.prod(kept))
+    assert (do.numpy()[:n] == 0).all() and (do.numpy()[n:] == 7).all()
+
+
 def test_reference_tensor_known_answers(ctx):
     """The reference's Tensor KATs through the backend ops: BroadcastingAdd
     (tensor_test.cpp:53-67, [2,3] + [1,3]), ElementwiseSubAndMul (:69-80),
