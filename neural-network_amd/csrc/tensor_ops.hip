@@ -136,6 +136,7 @@ constexpr int kKT = 32;
 // workgroups): 192 tiles 32.2 / 34.3 us (64 / 32), 128 tiles 30.8 / 23.8, 32
 // tiles 56 / 27, 1024 tiles 385 / 555.
 constexpr int kMatmulTiles64 = 160;
+constexpr int64_t kMatmulCols = 1 << 28;      // columns of one launch at most
 template <int TR, int TC, int THR>
 __global__ __launch_bounds__(THR) void matmul_kernel(
     const float *__restrict__ a, int64_t sa0, int64_t sa1,
@@ -557,15 +558,21 @@ void launch_matmul(hipStream_t st, const TensorView &a, const TensorView &b,
   NNHIP_REQUIRE(M < (1 << 30) && N < (1 << 30) && K < (1 << 30), kErrArg,
                 "matmul: extent too large");
   if (M == 0 || N == 0) return;
+  // 8 threads a column of the 64-wide tiles: the 2^32 threads of a launch along
+  // x are 2^29 columns, so wider products go out in parts
 #define NNHIP_MM(TR, TC, THR)                                                 \
-  hipLaunchKernelGGL((matmul_kernel<TR, TC, THR>),                            \
-                     dim3((unsigned)((N + 16 * TC - 1) / (16 * TC)),          \
-                          (unsigned)((M + THR / 16 * TR - 1) / (THR / 16 * TR))), \
-                     dim3(THR), 0, st, at(a), a.strides[0], a.strides[1],     \
-                     at(b), b.strides[0], b.strides[1], at_mut(out),          \
-                     out.strides[0], out.strides[1], (int)M, (int)N, (int)K)
-  if (((M + 63) / 64) * ((N + 63) / 64) >= kMatmulTiles64) NNHIP_MM(2, 4, 512);
-  else NNHIP_MM(1, 2, 512);
+  for (int64_t c0 = 0; c0 < N; c0 += kMatmulCols) {                           \
+    const int64_t n = std::min(N - c0, kMatmulCols);                          \
+    hipLaunchKernelGGL((matmul_kernel<TR, TC, THR>),                          \
+                       dim3((unsigned)((n + 16 * TC - 1) / (16 * TC)),        \
+                            (unsigned)((M + THR / 16 * TR - 1) / (THR / 16 * TR))), \
+                       dim3(THR), 0, st, at(a), a.strides[0], a.strides[1],   \
+                       at(b) + c0 * b.strides[1], b.strides[0], b.strides[1], \
+                       at_mut(out) + c0 * out.strides[1], out.strides[0],     \
+                       out.strides[1], (int)M, (int)n, (int)K);               \
+  }
+  if (((M + 63) / 64) * ((N + 63) / 64) >= kMatmulTiles64) NNHIP_MM(2, 4, 512)
+  else NNHIP_MM(1, 2, 512)
 #undef NNHIP_MM
   NNHIP_CHECK(hipGetLastError());
 }

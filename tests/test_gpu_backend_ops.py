@@ -177,6 +177,24 @@ def test_matmul_tiles_bit_exact(ctx, M, K, N):
         assert (got[M] == 7).all() and (got[:, N:] == 7).all()
 
 
+def test_matmul_columns_beyond_one_launch(ctx):
+    """One row times more columns than the threads of one launch cover, every
+    column the same one of b (stride 0): all of them are written, up to the
+    row's end and not past it."""
+    K, N = 33, 2 ** 29 + 70
+    a, b = np.arange(1, K + 1, dtype=np.float32), np.full(K, 0.5, np.float32)
+    da, db, do = dev(ctx, a), dev(ctx, b), ctx.array(shape=(N + 100,))
+    nnhip.call("nnhip_fill_f32", ctx.h, do.p, N + 100, 7.0)
+    nnhip.call("nnhip_matmul_f32", ctx.h, nnhip.view(da, (1, K)),
+               nnhip.view(db, (K, N), (1, 0)), nnhip.view(do, (1, N)))
+    got = np.empty(200, np.float32)
+    for at in (0, 2 ** 28 - 100, 2 ** 29 - 100, N - 100):
+        nnhip.call("nnhip_d2h", ctx.h, nnhip.ptr(got),
+                   np.ctypeslib.ctypes.c_void_p(do.p.value + 4 * at), got.nbytes)
+        assert (got[:min(200, N - at)] == 0.5 * K * (K + 1) / 2).all(), at
+    assert (got[100:] == 7).all()
+
+
 def test_matmul_known_answer_and_errors(ctx):
     """TensorTest.MatmulContiguous (tensor_test.cpp:82-94): [[1,2,3],[4,5,6]]
     . [[7,8],[9,10],[11,12]] = [[58,64],[139,154]]; shape errors carry the
