@@ -338,7 +338,8 @@ int nnhip_rope_kv_append_q8(nnhip_ctx *ctx, const float *qkv, int B, int S,
 /* nnhip_attention_kq over an int8 cache (layer.cpp:842-952, quantized
  * branches): element j of a cached row enters as (float)code * scale.
  * kcodes / vcodes [B][Hkv][cap][D], kscales / vscales [B][Hkv][cap].
- * Stream-ordered, with the scratch nnhip_attention_kq keeps in the context. */
+ * Returns with out written (the stream drained); its scratch is the one
+ * nnhip_attention_kq keeps in the context. */
 int nnhip_attention_kq_q8(nnhip_ctx *ctx, const float *q, const int8_t *kcodes,
                           const float *kscales, const int8_t *vcodes,
                           const float *vscales, int cap, const int32_t *pos0,

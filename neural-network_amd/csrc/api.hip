@@ -762,6 +762,9 @@ int nnhip_attention_kq_q8(nnhip_ctx *ctx, const float *q, const int8_t *kcodes,
     kv.sc_stride = (int64_t)Hkv * cap;
     nnhip::launch_attention(st, q, kv, B, S, H, Hkv, D, cap, pos0, 0, nullptr,
                             max_keys, ctx->part.p, pe, out);
+    // out is written and the operands are read when the call returns: callers
+    // may go on from another stream
+    NNHIP_CHECK(hipStreamSynchronize(st));
   });
 }
 

@@ -622,6 +622,30 @@ def test_attention_kq_q8(ctx, B, S, H, D, pos0, w4):
                           out.reshape(S, H * D), 1e-4, f"int8 attention seq {b}")
 
 
+def test_attention_kq_q8_returns_drained(ctx):
+    """nnhip_attention_kq_q8 returns with its output written: read through
+    another context (another stream) right away, behind milliseconds of
+    earlier work on its own, it is what a read on its own stream gives."""
+    B, S, H, D, cap = 2, 5, 4, 64, 400
+    rng = np.random.default_rng(8)
+    kv = [ctx.array(rng.integers(-127, 128, (B, H, cap, D)).astype(np.int8)) for _ in "kv"]
+    sc = [ctx.array((rng.random((B, H, cap)) * 0.03).astype(np.float32)) for _ in "kv"]
+    q = ctx.array(rng.standard_normal((B * S, H * D)).astype(np.float32))
+    pos, out = ctx.array(np.array([390, 7], np.int32)), ctx.array(np.zeros((B * S, H * D), np.float32))
+    n = 4096
+    x, w, y = (ctx.array(shape=(n, n)) for _ in range(3))
+    with nnhip.Context(0) as other:
+        for _ in range(3):
+            call("nnhip_linear_f32", ctx.h, x.p, n, n, w.p, x.p, n, y.p)
+        call("nnhip_attention_kq_q8", ctx.h, q.p, kv[0].p, sc[0].p, kv[1].p, sc[1].p,
+             cap, pos.p, B, S, H, H, D, out.p)
+        got = np.empty((B * S, H * D), np.float32)
+        call("nnhip_d2h", other.h, nnhip.ptr(got), out.p, got.nbytes)
+    want = out.numpy()
+    assert np.abs(want).min(1).max() > 0
+    np.testing.assert_array_equal(got, want)
+
+
 @pytest.mark.parametrize("rows,d", [(7, 64), (5, 1024), (3, 4096), (2, 100)])
 def test_layernorm(ctx, rows, d):
     rng = np.random.default_rng(d)
