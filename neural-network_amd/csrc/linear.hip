@@ -1143,10 +1143,16 @@ constexpr int kTallGroup = 8;   // row tiles that share a column tile in turn
 // An asm statement and not the builtin: behind the builtin the compiler waits
 // for every copy in flight before the next LDS read, whatever buffer it reads
 // (it has no register output; gemm_tall_kernel waits for the copies itself).
+// m0, which holds the LDS address, is named as clobbered, so that the compiler
+// keeps no m0 of its own across the statement; its warning is about registers
+// it reserves for a whole function, which m0 is not.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void tall_copy(const int8_t *src, uint32_t voff, uint32_t dst) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(dst), "v"(voff), "s"(src) : "memory");
+               :: "s"(dst), "v"(voff), "s"(src) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 template <int EPI>
 __global__ __launch_bounds__(kTallThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
