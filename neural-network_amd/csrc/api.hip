@@ -570,7 +570,7 @@ int nnhip_layernorm_linear_w8a32(nnhip_ctx *ctx, const float *h, int rows,
     const bool aligned = ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(gamma) |
                            reinterpret_cast<uintptr_t>(beta) |
                            reinterpret_cast<uintptr_t>(ln_out)) & 15) == 0;
-    if (aligned && nnhip::gemm_tall_shape(rows, K, N)) {
+    if (aligned && nnhip::gemm_tall_shape(rows, K, N, true)) {
       const int mpad = ctx_scratch(ctx, rows, K, N);
       nnhip::launch_swizzle_rows(st, codes, N, K, ctx->sw.p, false);
       nnhip::launch_layernorm(st, h, rows, K, gamma, beta, ln_out, ctx->limbs.p,

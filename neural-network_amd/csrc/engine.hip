@@ -581,7 +581,7 @@ void Model::forward(KVCache *cache, int b_off, const int32_t *ids,
     if (hd)
       launch_gemm_limb_hx(st, ws.limbs.p, ws.mpad, ws.hexp.p, R, d, d, ly.o.qs.p,
                           ly.o.s.p, ly.o.b.p, ws.x.p, d, ws.h.p, d, kEpiResid);
-    else if (merged && (R <= g_o_limb_rows || gemm_tall_shape(R, d, d)) &&
+    else if (merged && (R <= g_o_limb_rows || gemm_tall_shape(R, d, d, true)) &&
              use_limbs(ly.o, R))
       linear(ly.o, ws.ctx.p, d, R, false, ws.x.p, d, ws.h.p, d, kEpiResid);
     else if (merged && ly.o.quant && ly.o.qs.p && R >= kLimbMinRows &&

@@ -1135,7 +1135,7 @@ __global__ __launch_bounds__(kLdsThreads) void gemm_lds_kernel(
 // wide tile loads 23 bytes a clock and CU instead of 32.  Rest: 5.6 us a
 // launch outside the stages (first loads, the epilogue's 64 outputs a lane).
 // ---------------------------------------------------------------------------
-constexpr int kTallM = 128, kTallN = 256, kTallThreads = 512;
+constexpr int kTallThreads = 512;             // tile kTallM x kTallN (dispatch.hpp)
 constexpr int kTallStage = 40 * 1024, kTallBufs = 3;
 constexpr int kTallGroup = 8;   // row tiles that share a column tile in turn
 
@@ -1860,22 +1860,9 @@ void launch_gemm_operands(hipStream_t st, const float *x, int rows, int K,
 
 int g_limb_k8 = 512;
 
-// Where the 128 x 256-tile GEMM takes a digit-plane product over from the
-// other two: from 96 tiles on.  A tile takes 8 (K = 512) to 60 us (K = 4096)
-// however few there are, and 256 run at once; the other two GEMMs' time grows
-// with the rows throughout.  Measured, best of the other two against this one:
-// K = 1024, N = 8192: 128 tiles (512 rows) 25.7 / 24.2 us, 256 tiles 45.9 /
-// 28.8; N = 3072: 96 tiles 22.7 / 21.9, 48 tiles 13.4 / 21.4; K = 512, N =
-// 4096: 128 tiles 18.9 / 15.7, 64 tiles 11.3 / 14.0; K = 4096, N = 1024: 128
-// tiles 130 / 75, 64 tiles 68.3 / 67.4, 32 tiles 36.0 / 64.1.
-constexpr int kTallMinTiles = 96;
-bool gemm_tall_shape(int rows, int K, int N) {
-  const int64_t tiles = (int64_t)((rows + kTallM - 1) / kTallM) * ((N + kTallN - 1) / kTallN);
-  return tiles >= kTallMinTiles && K % 128 == 0 && N % 32 == 0;
-}
-static bool gemm_tall_takes(int rows, int K, int N, int64_t ldy, int epi,
-                            const RopeArgs *ra) {
-  return gemm_tall_shape(rows, K, N) && ldy < (1 << 23) && epi != kEpiTotals &&
+static bool gemm_tall_takes(int rows, int K, int N, bool vs_lds, int64_t ldy,
+                            int epi, const RopeArgs *ra) {
+  return gemm_tall_shape(rows, K, N, vs_lds) && ldy < (1 << 23) && epi != kEpiTotals &&
          !(epi == kEpiRope && ra && ra->kq);
 }
 
@@ -1919,7 +1906,7 @@ void launch_gemm_limb(hipStream_t st, const int8_t *limbs, int mpad,
   const bool q8 = epi == kEpiRope && rz.kq;
   NNHIP_REQUIRE(!q8 || gemm_limb_q8_ok(rz.D), kErrArg,
                 "gemm_limb: int8 KV append needs a power-of-two head dim <= 32");
-  if (gemm_tall_takes(rows, K, N, ldy, epi, ra)) {
+  if (gemm_tall_takes(rows, K, N, false, ldy, epi, ra)) {
     launch_gemm_tall(st, limbs, mpad, rexp, rows, K, N, wq, scale, bias, resid,
                      ldr, y, ldy, epi, rz);
     return;
@@ -2008,7 +1995,8 @@ void launch_gemm_lds(hipStream_t st, int mode, const int8_t *limbs, int mpad,
   NNHIP_REQUIRE(!ts || !ts->out || (gemm_lds_tile_width(K) > 0 && epi == kEpiBias),
                 kErrArg, "gemm_lds: tile statistics need K of 512 or 1024 and a bias epilogue");
   const TileStatsArgs tz = ts ? *ts : TileStatsArgs{};
-  if (mode == kAFromDigits && !tz.out && gemm_tall_takes(rows, K, N, ldy, epi, ra)) {
+  if (mode == kAFromDigits && !tz.out &&
+      gemm_tall_takes(rows, K, N, true, ldy, epi, ra)) {
     launch_gemm_tall(st, limbs, mpad, rexp, rows, K, N, wq, scale, bias, resid,
                      ldr, y, ldy, epi, rz);
     return;

@@ -2,6 +2,8 @@
 // libnnhip.so.  Nothing here is part of the C ABI (include/nnhip.h is).
 #pragma once
 
+#include "dispatch.hpp"
+
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -403,9 +405,8 @@ void launch_gemm_operands(hipStream_t st, const float *x, int rows, int K,
                           int8_t *limbs, int mpad, int *rexp,
                           const int8_t *codes, int N, int8_t *sw);
 bool gemm_limb_q8_ok(int D);
-// whether a product over digit planes is tall enough for the 128 x 256-tile
-// GEMM (launch_gemm_limb and launch_gemm_lds then run that one)
-bool gemm_tall_shape(int rows, int K, int N);
+// launch_gemm_limb and launch_gemm_lds run the 128 x 256-tile GEMM where
+// gemm_tall_shape (dispatch.hpp) says so
 void launch_gemm_limb(hipStream_t st, const int8_t *limbs, int mpad,
                       const int *rexp, int rows, int K, int N,
                       const int8_t *wq, const float *scale, const float *bias,

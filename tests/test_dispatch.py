@@ -1,0 +1,41 @@
+"""The rules on sizes that choose between kernels (csrc/dispatch.hpp), asked on
+the CPU: every shape below was timed with both kernels on an MI355X, and the
+rule takes the faster one (a tie may go either way)."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+from gpu_util import ROOT
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    lib = tmp_path_factory.mktemp("dispatch") / "dispatch_rules.so"
+    subprocess.check_call(
+        ["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC",
+         "-I", os.path.join(ROOT, "neural-network_amd", "csrc"),
+         os.path.join(ROOT, "tests", "cpp", "dispatch_rules.cpp"), "-o", str(lib)])
+    return ctypes.CDLL(str(lib))
+
+
+@pytest.mark.parametrize("vs_lds,rows,K,N,tall", [
+    # against the LDS-resident GEMM: wide products of few rows stay there
+    (1, 16, 1024, 32000, 0), (1, 64, 1024, 32000, 0), (1, 96, 1024, 32000, 0),
+    (1, 128, 1024, 32000, 1), (1, 192, 1024, 32000, 1), (1, 288, 1024, 32000, 1),
+    (1, 96, 512, 32000, 0), (1, 128, 512, 32000, 1), (1, 64, 256, 32768, 0),
+    (1, 96, 128, 32768, 0), (1, 128, 128, 32768, 1), (1, 96, 1024, 24576, 0),
+    (1, 128, 1024, 24576, 1), (1, 16, 1024, 200000, 0), (1, 512, 1024, 8192, 1),
+    (1, 1024, 1024, 3072, 1), (1, 512, 1024, 3072, 0), (1, 8192, 1024, 8192, 1),
+    # against the digit-plane GEMM
+    (0, 64, 4096, 32000, 0), (0, 128, 4096, 32000, 1), (0, 192, 4096, 12288, 0),
+    (0, 256, 4096, 12288, 1), (0, 288, 4096, 8192, 0), (0, 384, 4096, 8192, 1),
+    (0, 4096, 4096, 1024, 1), (0, 64, 2048, 32768, 0), (0, 192, 2048, 12288, 0),
+    (0, 256, 2048, 12288, 1), (0, 512, 2048, 6144, 1), (0, 32, 1024, 32000, 0),
+    (0, 128, 1024, 32000, 1), (0, 32, 512, 32768, 0), (0, 64, 512, 32768, 1),
+    (0, 64, 128, 32768, 1),
+    # what the kernel does not take
+    (1, 4096, 1024, 4104, 0), (0, 4096, 960, 4096, 0)])
+def test_tall_gemm(rules, vs_lds, rows, K, N, tall):
+    assert rules.gemm_tall_shape(rows, K, N, vs_lds) == tall
