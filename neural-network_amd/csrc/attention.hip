@@ -29,7 +29,6 @@ constexpr int kMaxQ = 8;       // queries per workgroup
 // attn_short_q: launches of fewer (sequence, head) pairs than this take
 // their queries in blocks of g_attn_short_q
 constexpr int kAttnShortUnits = 64;
-constexpr int kPromptQ = 20, kPromptGrid = 160;   // attn_prompt_kernel (prompt_shape)
 constexpr int kMaxD = 64;      // head dim handled by the attention kernel
 
 // Embedding gather (cpu_backend.cpp:1020-1025): ids outside [0, vocab) read
@@ -742,7 +741,7 @@ __global__ __launch_bounds__(kWave * W, W == 4 ? 2 : 1) void attn_kernel(
 
 // ---------------------------------------------------------------------------
 // Prompt attention: 32 queries of one (head, sequence) per workgroup on the
-// fp32 MFMA (prompts; the rule is at prompt_shape).  The W
+// fp32 MFMA (prompts; the rule is attention_prompt_shape, dispatch.hpp).  The W
 // waves of a workgroup take the visible 32-key chunks in turn (chunk w, w +
 // W, ...), each with its own online softmax, and merge in LDS as the merged
 // split-K workgroups do; nothing passes between them before that, so the
@@ -774,7 +773,7 @@ __global__ __launch_bounds__(kWave * W, W == 4 ? 2 : 1) void attn_kernel(
 // 300 cached ones: 39.9 -> 31.3.
 // ---------------------------------------------------------------------------
 typedef float attn_v16f __attribute__((ext_vector_type(16)));
-constexpr int kPromptTile = 32, kPromptWaves = 4;
+constexpr int kPromptWaves = 4;                // tiles of kPromptTile queries
 
 template <int DL, bool Q8, bool MS>
 __global__ __launch_bounds__(kWave * kPromptWaves, 2) void attn_prompt_kernel(
@@ -1409,17 +1408,13 @@ bool attention_merged(int D, int max_keys) {
          max_keys <= kMergedWaves * kMergedChunks * kChunk;
 }
 
-// Launches of the prompt kernel: tiles that are not mostly empty, and enough
-// of them.  16 positions a sequence take as long either way and 20 are faster
-// here (16 x 16 heads after 300 keys: 19.8 / 19.7 us, 27.1 -> 20.3); below
-// 160 workgroups the MFMAs of a few CUs would carry the launch that the
-// split-K kernel spreads over the chip (4 heads x 22 tiles: 23.2 us there,
-// 26.6 here; 8 x 22: 22.3 -> 17.2).  Its loads are 16 bytes wide at every head
-// dim and its offsets in a head's rows 32 bits; what is not aligned for them,
-// or longer, stays with the split-K kernel.
-static bool prompt_shape(const float *q, const KvSrc &kv, int B, int S, int H, int D, int cap) {
-  return S >= kPromptQ &&
-         (int64_t)B * H * ((S + kPromptTile - 1) / kPromptTile) >= kPromptGrid && (int64_t)cap * D < (1 << 29) &&
+// Launches of the prompt kernel: the sizes it is the faster on, and what its
+// loads can take.  They are 16 bytes wide at every head dim and its offsets in
+// a head's rows 32 bits; what is not aligned for them, or longer, stays with
+// the split-K kernel.
+static bool prompt_shape(const float *q, const KvSrc &kv, int B, int S, int H, int D, int cap,
+                         int max_keys) {
+  return attention_prompt_shape(B, S, H, D, kv.q8, max_keys) && (int64_t)cap * D < (1 << 29) &&
          ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kv.k) |
            reinterpret_cast<uintptr_t>(kv.v)) & 15) == 0 &&
          (kv.seq_stride & (kv.q8 && D == 64 ? 15 : 3)) == 0;
@@ -1451,7 +1446,7 @@ bool launch_attention(hipStream_t st, const float *q, const KvSrc &kv, int B,
   const bool merged = attention_merged(D, max_keys);
   NNHIP_REQUIRE(!hexp || (limbs && D == kWave && (H * D) % 128 == 0 && B * S <= mpad),
                 kErrArg, "attention: head digits need D == 64, H*D % 128 == 0");
-  if (prompt_shape(q, kv, B, S, H, D, cap)) {
+  if (prompt_shape(q, kv, B, S, H, D, cap, max_keys)) {
     const dim3 grid(B * H, (S + kPromptTile - 1) / kPromptTile);
     int8_t *hl = merged && hexp ? limbs : nullptr;
 #define NNHIP_ATTN_MS(DL, Q8, MS)                                             \

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 namespace nnhip {
@@ -32,6 +33,39 @@ inline bool gemm_tall_shape(int rows, int K, int N, bool vs_lds) {
   const int64_t least = vs_lds ? kFull : std::min(kFull, ((int64_t)1 << 20) + 1024 * (int64_t)K);
   return K % 128 == 0 && N % 32 == 0 && tiles >= kMinTiles &&
          rows >= (vs_lds ? kTallM : kTallM / 2) && (int64_t)rows * N >= least;
+}
+
+// Launches of the prompt attention kernel, tiles of 32 queries of one
+// (sequence, head), against the split-K kernel, 8 queries a workgroup, for
+// caches of up to max_keys keys.  16 positions a sequence take as long either
+// way and 20 are faster in tiles (16 x 16 heads after 300 keys: 19.8 / 19.7 us,
+// 27.1 -> 20.3); below 160 tiles the MFMAs of a few CUs would carry the launch
+// that the split-K kernel spreads over the chip (4 heads x 22 tiles: 23.2 us
+// there, 26.6 here; 8 x 22: 22.3 -> 17.2).
+// Over long caches both are bound by their products, the tiles' including
+// those of the empty rows of a tile and of the CUs without a tile in the last
+// round of 256: `waste` is the tiles' products over the split-K kernel's.  With
+// `share` the time of a tile's product in the split-K kernel's, the tiles are
+// the faster while waste x share is below 1 (1.05: ties).  Measured shares of
+// waste 1.6 to 2.6 at 1024 / 2048 / 4096 / 8192 keys: 8 dims 0.45 / 0.56 / 0.60 /
+// 0.68, 16 dims 0.43 / 0.51 / 0.54 / 0.57, 32 dims 0.40 / 0.39 / 0.40 / 0.46,
+// 40 dims 0.39 / 0.46 / 0.49 / 0.51, 64 dims 0.39 / 0.37 / 0.36 / 0.39, over int8
+// rows up to 0.43.  160 pairs x 40 positions over 16000 keys (waste 2.6),
+// split-K / tiles: 16 dims 200 / 298 us, 40 dims 477 / 590, 64 dims of int8 rows
+// 612 / 703; over 4000 keys 64 dims 203 / 177.
+constexpr int kPromptTile = 32;
+inline bool attention_prompt_shape(int B, int S, int H, int D, bool q8, int max_keys) {
+  const int64_t pairs = (int64_t)B * H;
+  const int64_t tiles = pairs * ((S + kPromptTile - 1) / kPromptTile);
+  if (S < 20 || tiles < 160) return false;
+  const double waste = (double)((tiles + 255) / 256 * 256 * kPromptTile) /
+                       (double)(pairs * ((S + 7) / 8) * 8);
+  const double doublings = std::max(-1.0, std::log2(max_keys / 1024.0));
+  const double share = D <= 16               ? 0.45 + 0.08 * doublings
+                       : D == 64 && !q8      ? 0.40
+                       : D == 64 || D == 32  ? 0.40 + 0.02 * doublings
+                                             : 0.40 + 0.04 * doublings;
+  return waste * share <= 1.05;
 }
 
 }  // namespace nnhip

@@ -5,4 +5,7 @@ extern "C" {
 int gemm_tall_shape(int rows, int K, int N, int vs_lds) {
   return nnhip::gemm_tall_shape(rows, K, N, vs_lds != 0);
 }
+int attention_prompt_shape(int B, int S, int H, int D, int q8, int max_keys) {
+  return nnhip::attention_prompt_shape(B, S, H, D, q8 != 0, max_keys);
+}
 }

@@ -39,3 +39,19 @@ def rules(tmp_path_factory):
     (1, 4096, 1024, 4104, 0), (0, 4096, 960, 4096, 0)])
 def test_tall_gemm(rules, vs_lds, rows, K, N, tall):
     assert rules.gemm_tall_shape(rows, K, N, vs_lds) == tall
+
+
+@pytest.mark.parametrize("B,S,H,D,q8,keys,prompt", [
+    # long caches behind tiles of which much is empty, or fewer than the CUs
+    (40, 40, 4, 16, 0, 16000, 0), (40, 40, 4, 16, 0, 4096, 0), (40, 20, 4, 16, 0, 8192, 0),
+    (40, 40, 4, 16, 0, 512, 1), (40, 64, 4, 16, 0, 2048, 1), (20, 40, 8, 8, 0, 2048, 0),
+    (20, 40, 8, 40, 0, 4096, 0), (20, 40, 8, 40, 0, 1024, 1), (20, 64, 8, 40, 0, 8192, 1),
+    (20, 40, 8, 32, 0, 8192, 0), (20, 28, 8, 32, 0, 8192, 1), (20, 36, 8, 24, 0, 8192, 0),
+    (5, 40, 32, 64, 1, 16000, 0), (5, 40, 32, 64, 1, 1024, 1), (5, 64, 32, 64, 1, 8192, 1),
+    (10, 40, 16, 64, 0, 4000, 1), (10, 20, 16, 64, 0, 8000, 1), (128, 36, 8, 8, 0, 2048, 1),
+    # prompts proper
+    (4, 1000, 16, 64, 0, 1024, 1), (8, 300, 8, 32, 1, 4096, 1), (4, 1000, 16, 8, 0, 16384, 1),
+    # too short, too few
+    (64, 16, 16, 64, 0, 512, 0), (1, 100, 16, 64, 0, 512, 0), (1, 320, 16, 64, 0, 512, 1)])
+def test_prompt_attention(rules, B, S, H, D, q8, keys, prompt):
+    assert rules.attention_prompt_shape(B, S, H, D, q8, keys) == prompt
