@@ -68,4 +68,30 @@ inline bool attention_prompt_shape(int B, int S, int H, int D, bool q8, int max_
   return waste * share <= 1.05;
 }
 
+// fp32 products (and int8 ones of shapes the digit GEMMs do not take).  The
+// fp32 MFMA GEMM takes the GEMV over from 16 rows and 90000 outputs on: the
+// GEMV runs at about 20 TFLOP/s, the GEMM costs 7 ns per entry of K and wave
+// whatever the size, so the line does not depend on K.  Measured (GEMV /
+// GEMM): 64 x 2048 at K = 512 11.1 / 7.9 us, 64 x 512 at K = 2048 8.5 / 18.4,
+// 128 x 512 at K = 512 6.7 / 7.8, 128 x 3072 at K = 1024 54 / 18.5.
+inline bool gemm_f32_shape(int rows, int N) {
+  return rows >= 16 && (int64_t)rows * N >= 90000;
+}
+
+// Its tile, 64 x 64 (0) or 32 x 32 with K over 4 or 8 waves (returned).  64 x 64
+// when there are enough of them and more than half of their rows are filled
+// (2048 x 4096 at K = 1024, 2048 tiles: 175 us with 64 x 64, 254 with 32 x 32;
+// 512 x 1024, 128 tiles: 32 / 19; 16 x 62501 at K = 1024, int8 codes: 96 / 63,
+// GEMV 77).  8 waves when their workgroups run at once (64 x 1024 at K = 4096:
+// 41 us over 4 waves, 34 over 8; 16 x 5626, 176 tiles, at K = 4096, int8 codes:
+// 39 / 30, GEMV 32; 16 x 12501, 391 tiles: 55 / 58).  K below 64 is too short to
+// split (256 x 352, 64 x 64 / 4 waves: K = 64 5.2 / 4.6 us, K = 252 10.1 / 5.6,
+// GEMV 5.8).
+inline int gemm_f32_waves(int rows, int K, int N) {
+  const int64_t t64 = (int64_t)((rows + 63) / 64) * ((N + 63) / 64);
+  const int64_t t32 = (int64_t)((rows + 31) / 32) * ((N + 31) / 32);
+  if (K < 64 || (t64 >= 448 && rows > 32)) return 0;
+  return t32 > 256 || K < 512 ? 4 : 8;
+}
+
 }  // namespace nnhip

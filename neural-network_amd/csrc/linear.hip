@@ -1723,13 +1723,6 @@ int g_gemm_wide = 1;
 // 1: int8 GEMVs with K of 256-4096 use 128-bit code loads (gemv16_kernel)
 int g_gemv16 = 1;
 
-// The fp32 MFMA GEMM takes a GEMV over from 16 rows and 90000 outputs on: the
-// GEMV runs at about 20 TFLOP/s, the GEMM costs 7 ns per entry of K and wave
-// whatever the size, so the line does not depend on K.  Measured (GEMV /
-// GEMM): 64 x 2048 at K = 512 11.1 / 7.9 us, 64 x 512 at K = 2048 8.5 / 18.4,
-// 128 x 512 at K = 512 6.7 / 7.8, 128 x 3072 at K = 1024 54 / 18.5.
-constexpr int kF32MinRows = 16;
-constexpr int64_t kF32MinOutputs = 90000;
 static void launch_gemm_f32(hipStream_t st, const float *x, int64_t ldx, int rows,
                             int K, int N, const int8_t *wq, const float *wf,
                             const float *scale, const float *bias,
@@ -1748,13 +1741,9 @@ static void launch_gemm_f32(hipStream_t st, const float *x, int64_t ldx, int row
                          ldx, rows, K, N, wq, wf, scale, bias, resid, ldr, y, ldy, \
                          epi, ntm, ntn, ra);                                  \
   }
-  // 64 x 64 tiles when there are enough of them, else 32 x 32 ones with K over
-  // 4 or 8 waves (2048 x 4096 at K = 1024, 2048 tiles: 175 us with 64 x 64,
-  // 254 with 32 x 32; 512 x 1024, 128 tiles: 32 / 19; 64 x 1024 at K = 4096,
-  // 16 tiles: 41 us over 4 waves, 34 over 8; K below 256 is too short to split)
-  const int64_t t64 = (int64_t)((rows + 63) / 64) * ((N + 63) / 64);
-  if (t64 >= 448 || K < 256) NNHIP_GF(2, 2, 1)
-  else if (t64 > 64 || K < 512) NNHIP_GF(1, 1, 4)
+  const int waves = gemm_f32_waves(rows, K, N);
+  if (waves == 0) NNHIP_GF(2, 2, 1)
+  else if (waves == 4) NNHIP_GF(1, 1, 4)
   else NNHIP_GF(1, 1, 8)
 #undef NNHIP_GF
   NNHIP_CHECK(hipGetLastError());
@@ -1774,7 +1763,7 @@ void launch_gemv(hipStream_t st, const float *x, int64_t ldx, int rows, int K,
   NNHIP_REQUIRE(!(ra && ra->kq), kErrArg,
                 "gemv: no int8 KV append in this epilogue (use rope_kv_q8)");
   const RopeArgs rz = ra ? *ra : RopeArgs{};
-  if (!lz.g && rows >= kF32MinRows && (int64_t)rows * N >= kF32MinOutputs) {
+  if (!lz.g && gemm_f32_shape(rows, N)) {
     launch_gemm_f32(st, x, ldx, rows, K, N, wq, wf, scale, bias, resid, ldr, y,
                     ldy, epi, rz);
     return;

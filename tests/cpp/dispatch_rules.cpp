@@ -8,4 +8,6 @@ int gemm_tall_shape(int rows, int K, int N, int vs_lds) {
 int attention_prompt_shape(int B, int S, int H, int D, int q8, int max_keys) {
   return nnhip::attention_prompt_shape(B, S, H, D, q8 != 0, max_keys);
 }
+int gemm_f32_shape(int rows, int N) { return nnhip::gemm_f32_shape(rows, N); }
+int gemm_f32_waves(int rows, int K, int N) { return nnhip::gemm_f32_waves(rows, K, N); }
 }

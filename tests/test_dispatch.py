@@ -55,3 +55,20 @@ def test_tall_gemm(rules, vs_lds, rows, K, N, tall):
     (64, 16, 16, 64, 0, 512, 0), (1, 100, 16, 64, 0, 512, 0), (1, 320, 16, 64, 0, 512, 1)])
 def test_prompt_attention(rules, B, S, H, D, q8, keys, prompt):
     assert rules.attention_prompt_shape(B, S, H, D, q8, keys) == prompt
+
+
+@pytest.mark.parametrize("rows,K,N,waves", [
+    # a short K is split over 4 waves all the same
+    (16, 252, 5626, 4), (256, 252, 352, 4), (64, 64, 2032, 4), (512, 128, 391, 4),
+    (512, 252, 4096, 0), (1000, 60, 91, 0),
+    # few rows: 32 x 32 tiles, which are counted as such
+    (16, 4096, 5626, 8), (16, 2048, 5626, 8), (16, 1024, 8126, 8), (16, 1024, 12501, 4),
+    (24, 4096, 3751, 8), (32, 2048, 31251, 4), (16, 1024, 62501, 4), (33, 1024, 62501, 0),
+    (333, 772, 1544, 4), (64, 4096, 1024, 8), (512, 1024, 1024, 4), (2048, 1024, 4096, 0)])
+def test_f32_gemm_tiles(rules, rows, K, N, waves):
+    assert rules.gemm_f32_waves(rows, K, N) == waves
+
+
+def test_f32_gemm_from_90000_outputs(rules):
+    assert rules.gemm_f32_shape(16, 5625) and not rules.gemm_f32_shape(15, 60000)
+    assert not rules.gemm_f32_shape(16, 5624) and rules.gemm_f32_shape(90000, 65536)

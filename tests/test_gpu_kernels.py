@@ -986,9 +986,10 @@ def test_tall_forward_matches_short_batches(ctx, B, S, q8):
 
 @pytest.mark.parametrize("q8", [False, True])
 @pytest.mark.parametrize("rows,K,N", [
-    # 64 x 64 tiles, K below 256: remainders of rows, columns and K steps
-    (1407, 64, 64), (1000, 4, 91), (301, 252, 301),
-    # 32 x 32 tiles over 4 waves, then over 8 (64 tiles or fewer)
+    # 64 x 64 tiles, K below 64: remainders of rows, columns and K steps
+    (1000, 60, 91), (1000, 4, 91),
+    # 32 x 32 tiles over 4 waves, K from 64 on, then over 8 (256 tiles or fewer)
+    (1407, 64, 64), (301, 252, 301),
     (333, 260, 1544), (500, 772, 1001), (40, 508, 2251), (97, 1000, 929),
     (16, 4096, 5625), (352, 4092, 257),
     # 64 x 64 tiles of a large product
