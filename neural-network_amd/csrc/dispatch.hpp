@@ -94,4 +94,21 @@ inline int gemm_f32_waves(int rows, int K, int N) {
   return t32 > 256 || K < 512 ? 4 : 8;
 }
 
+// Sums of the backend that run with a thread an output (sum_short_kernel) and
+// not in tiles through LDS (sum_kernel): short ones, longer where neighbouring
+// outputs are neighbours in memory (along_r false), and there of any length from
+// 65536 outputs on, whose threads fill the chip; along the sums also those that
+// leave much of a 32-entry tile empty.  Measured, tiles / threads, in us (a
+// thread an output with one load at a time, before both):
+//   along the outputs: 2 x 1 M 25.2 / 7.5 (8.5), 32 x 8192 6.2 / 5.8 (12.9), 64 x
+//     8192 5.5 / 6.1 (22), 40 x 131072 17.8 / 5.8 (16.5), 64 x 262144 30.6 / 12.1
+//     (41), 300 x 131072 169 / 31 (148), 1000 x 16384 47 / 74 (439)
+//   along the sums: 8 x 1 M 28.2 / 17.1 (19.5), 12 x 1 M 29.7 / 19.6 (27.4), 16 x
+//     1 M 31.6 / 32.6 (40), 17 x 262144 14.7 / 8.3 (12.5), 24 x 1 M 59 / 51 (201),
+//     32 x 1 M 67 / 89 (531), 64 x 262144 27.6 / 44.8 (71)
+inline bool sum_short_shape(int64_t n_out, int64_t n_red, bool along_r) {
+  if (!along_r) return n_red <= 32 || n_out >= 65536;
+  return n_red <= 12 || (n_red > 16 && n_red <= 24 && n_out >= 131072);
+}
+
 }  // namespace nnhip

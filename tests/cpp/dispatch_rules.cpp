@@ -10,4 +10,7 @@ int attention_prompt_shape(int B, int S, int H, int D, int q8, int max_keys) {
 }
 int gemm_f32_shape(int rows, int N) { return nnhip::gemm_f32_shape(rows, N); }
 int gemm_f32_waves(int rows, int K, int N) { return nnhip::gemm_f32_waves(rows, K, N); }
+int sum_short_shape(long long n_out, long long n_red, int along_r) {
+  return nnhip::sum_short_shape(n_out, n_red, along_r != 0);
+}
 }

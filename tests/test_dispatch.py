@@ -72,3 +72,15 @@ def test_f32_gemm_tiles(rules, rows, K, N, waves):
 def test_f32_gemm_from_90000_outputs(rules):
     assert rules.gemm_f32_shape(16, 5625) and not rules.gemm_f32_shape(15, 60000)
     assert not rules.gemm_f32_shape(16, 5624) and rules.gemm_f32_shape(90000, 65536)
+
+
+@pytest.mark.parametrize("n_out,n_red,along_sums,short", [
+    (1 << 20, 2, 0, 1), (1 << 20, 1, 1, 1), (1 << 20, 32, 0, 1), (1 << 20, 64, 0, 1),
+    (131072, 300, 0, 1), (8192, 32, 0, 1), (8192, 64, 0, 0), (16384, 1000, 0, 0),
+    (1 << 20, 8, 1, 1), (1 << 20, 12, 1, 1), (1 << 20, 16, 1, 0), (262144, 17, 1, 1),
+    (1 << 20, 24, 1, 1), (1 << 20, 32, 1, 0), (262144, 64, 1, 0),
+    (100, 1024, 0, 0), (1024, 1024, 1, 0), (1, 1 << 20, 1, 0), (16, 4, 1, 1)])
+def test_short_sums(rules, n_out, n_red, along_sums, short):
+    f = rules.sum_short_shape
+    f.argtypes = [ctypes.c_longlong, ctypes.c_longlong, ctypes.c_int]
+    assert f(n_out, n_red, along_sums) == short

@@ -261,6 +261,36 @@ def test_sum_tiles_bit_exact(ctx, shape, axes, perm):
     np.testing.assert_array_equal(do.numpy().reshape(want.shape), want)
 
 
+@pytest.mark.parametrize("shape,axes,perm", [
+    # along the outputs: 1 to 32 entries, and more over 65536 outputs and more
+    ((1, 777), (0,), None), ((7, 1000), (0,), None), ((8, 3, 500), (0,), None),
+    ((32, 1030), (0,), None), ((33, 65536), (0,), None), ((41, 70001), (0,), None),
+    # along the sums, up to 12; two reduced dims; a transposed input
+    ((999, 12), (1,), None), ((999, 9), (1,), None), ((2, 700, 4), (0, 2), None),
+    ((3, 50, 2, 6), (0, 2), (3, 1, 0, 2)), ((500, 11), (1,), (1, 0)),
+    ((131072, 17), (1,), None),
+    # at the line on either side of it
+    ((999, 13), (1,), None), ((33, 65535), (0,), None), ((33, 1030), (0,), None)])
+def test_sum_short_bit_exact(ctx, shape, axes, perm):
+    """Sums with a thread an output (few entries, or many outputs): remainders
+    of the eight entries requested together and of the workgroup, kept and
+    dropped dims, into a strided output; the ascending-order float32 sum bit
+    for bit, the entries between the outputs untouched."""
+    rng = np.random.default_rng(len(shape) + shape[0])
+    x = rng.standard_normal(shape).astype(np.float32)
+    x.flat[3] = -0.0
+    _, vx = strided(ctx, x, perm) if perm else (None, nnhip.view(dev(ctx, x)))
+    ax = (np.ctypeslib.ctypes.c_int64 * len(axes))(*axes)
+    for keep in (True, False):
+        want = serial_sum(x, axes, keep)
+        do = ctx.array(np.full((want.size, 2), 7, np.float32))
+        st = [2 * int(np.prod(want.shape[i + 1:])) for i in range(want.ndim)]
+        nnhip.call("nnhip_sum_f32", ctx.h, vx, nnhip.view(do, want.shape, st),
+                   ax, len(axes))
+        np.testing.assert_array_equal(do.numpy()[:, 0].reshape(want.shape), want)
+        assert (do.numpy()[:, 1] == 7).all()
+
+
 @pytest.mark.parametrize("shape,axes,strides", [
     ((2 ** 31 + 9, 0), (0, 1), (0, 1)), ((0, 2 ** 31, 3), (0, 1), (0, 0, 1)),
     ((70000, 70000, 0), (0, 1, 2), (70000, 1, 1))])
