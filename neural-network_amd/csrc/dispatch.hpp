@@ -94,6 +94,22 @@ inline int gemm_f32_waves(int rows, int K, int N) {
   return t32 > 256 || K < 512 ? 4 : 8;
 }
 
+// Backend products that run on matmul_short_kernel and not on matmul_kernel:
+// those with too little K to fill the latter's steps of 32, over many tiles
+// (of 64 x 64): the fewer the shorter the K and the emptier the tiles.
+// Measured, matmul_kernel / short, in us:
+//   up to 32 rows or columns: 1 x 4 x 65536 6.4 / 6.0, 1 x 16 x 100000 12.5 / 9.3, 8 x
+//     4 x 131072 10.1 / 6.3, 8 x 24 x 131072 17.2 / 14.4, 8 x 32 x 131072 17.2 / 17.4,
+//     32 x 12 x 1 M 86 / 61, 8 x 40 x 1 M 151 / 127, 8 x 64 x 1 M 193 / 215
+//   up to 64: 64 x 12 x 262144 28.1 / 31.4, 64 x 12 x 1 M 145 / 123
+//   more: 4096 x 4 x 16384 73 / 89, 32768 x 4 x 4096 193 / 176, 100 x 12 x 1 M 189 /
+//     168, 131072 x 4 x 1000 267 / 189, 131072 x 32 x 1000 352 / 393
+inline bool matmul_short_shape(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), side = std::min(M, N);
+  if (K >= 32) return K < 64 && side <= 32 && tiles >= 8192;
+  return tiles >= (side <= 32 ? 64 * std::max<int64_t>(K, 16) : side <= 64 ? 16384 : 32768);
+}
+
 // Sums of the backend that run with a thread an output (sum_short_kernel) and
 // not in tiles through LDS (sum_kernel): short ones, longer where neighbouring
 // outputs are neighbours in memory (along_r false), and there of any length from

@@ -228,6 +228,55 @@ __global__ __launch_bounds__(THR) void matmul_kernel(
     }
 }
 
+// Products with a short K and many tiles, or few rows or columns: 64 x 64 output
+// tiles, a 16 x 16 thread block, each thread 4 x 4 outputs; K staged through
+// LDS 16 at a time.  Its 8 KB of LDS let as many workgroups share a CU as its
+// registers do, which hides the operands' latency where a tile has little to
+// multiply (matmul_kernel: 37 KB and 8 waves a workgroup).  Bound: the tiles'
+// first loads and the stores.  1 x 1 x 1 M 18 us (matmul_kernel 47), 8 x 8 x 1 M
+// 38 (70), 32 x 12 x 1 M 61 (86), 131072 x 4 x 1000 189 (267).
+constexpr int kShortT = 64, kShortK = 16;
+__global__ __launch_bounds__(kBlock) void matmul_short_kernel(
+    const float *__restrict__ a, int64_t sa0, int64_t sa1,
+    const float *__restrict__ b, int64_t sb0, int64_t sb1,
+    float *__restrict__ o, int64_t so0, int64_t so1, int M, int N, int K) {
+  __shared__ float As[kShortK][kShortT + 1];
+  __shared__ float Bs[kShortK][kShortT + 1];
+  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
+  const int r0 = blockIdx.y * kShortT, c0 = blockIdx.x * kShortT;
+  float acc[4][4] = {};
+  for (int k0 = 0; k0 < K; k0 += kShortK) {
+    for (int e = threadIdx.x; e < kShortK * kShortT; e += kBlock) {
+      const int kk = e / kShortT, mm = e % kShortT;
+      const int r = r0 + mm, c = c0 + mm, k = k0 + kk;
+      As[kk][mm] = (r < M && k < K) ? a[r * sa0 + k * sa1] : 0.0f;
+      Bs[kk][mm] = (c < N && k < K) ? b[k * sb0 + c * sb1] : 0.0f;
+    }
+    __syncthreads();
+    const int kn = min(kShortK, K - k0);
+    for (int kk = 0; kk < kn; ++kk) {
+      float av[4], bv[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) av[i] = As[kk][ty * 4 + i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bv[j] = Bs[kk][tx * 4 + j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = acc[i][j] + av[i] * bv[j];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = r0 + ty * 4 + i, c = c0 + tx * 4 + j;
+      if (r < M && c < N) o[r * so0 + c * so1] = acc[i][j];
+    }
+}
+
 // Sum over axes.  Each output adds its inputs in ascending input index (a
 // serial chain, so no output's sum is split): a workgroup owns OT outputs,
 // all of its threads bring tiles of RC reduced entries x OT outputs into LDS
@@ -598,19 +647,21 @@ void launch_matmul(hipStream_t st, const TensorView &a, const TensorView &b,
   if (M == 0 || N == 0) return;
   // 8 threads a column of the 64-wide tiles: the 2^32 threads of a launch along
   // x are 2^29 columns, so wider products go out in parts
-#define NNHIP_MM(TR, TC, THR)                                                 \
+#define NNHIP_MM(kernel, MT, NT, THR)                                         \
   for (int64_t c0 = 0; c0 < N; c0 += kMatmulCols) {                           \
     const int64_t n = std::min(N - c0, kMatmulCols);                          \
-    hipLaunchKernelGGL((matmul_kernel<TR, TC, THR>),                          \
-                       dim3((unsigned)((n + 16 * TC - 1) / (16 * TC)),        \
-                            (unsigned)((M + THR / 16 * TR - 1) / (THR / 16 * TR))), \
+    hipLaunchKernelGGL((kernel),                                              \
+                       dim3((unsigned)((n + NT - 1) / NT),                    \
+                            (unsigned)((M + MT - 1) / MT)),                   \
                        dim3(THR), 0, st, at(a), a.strides[0], a.strides[1],   \
                        at(b) + c0 * b.strides[1], b.strides[0], b.strides[1], \
                        at_mut(out) + c0 * out.strides[1], out.strides[0],     \
                        out.strides[1], (int)M, (int)n, (int)K);               \
   }
-  if (((M + 63) / 64) * ((N + 63) / 64) >= kMatmulTiles64) NNHIP_MM(2, 4, 512)
-  else NNHIP_MM(1, 2, 512)
+  if (matmul_short_shape(M, N, K)) NNHIP_MM(matmul_short_kernel, kShortT, kShortT, kBlock)
+  else if (((M + 63) / 64) * ((N + 63) / 64) >= kMatmulTiles64)
+    NNHIP_MM((matmul_kernel<2, 4, 512>), 64, 64, 512)
+  else NNHIP_MM((matmul_kernel<1, 2, 512>), 32, 32, 512)
 #undef NNHIP_MM
   NNHIP_CHECK(hipGetLastError());
 }

@@ -13,4 +13,7 @@ int gemm_f32_waves(int rows, int K, int N) { return nnhip::gemm_f32_waves(rows, 
 int sum_short_shape(long long n_out, long long n_red, int along_r) {
   return nnhip::sum_short_shape(n_out, n_red, along_r != 0);
 }
+int matmul_short_shape(long long M, long long N, long long K) {
+  return nnhip::matmul_short_shape(M, N, K);
+}
 }

@@ -84,3 +84,16 @@ def test_short_sums(rules, n_out, n_red, along_sums, short):
     f = rules.sum_short_shape
     f.argtypes = [ctypes.c_longlong, ctypes.c_longlong, ctypes.c_int]
     assert f(n_out, n_red, along_sums) == short
+
+
+@pytest.mark.parametrize("M,K,N,short", [
+    (1, 1, 1 << 20, 1), (1 << 20, 8, 1, 1), (1, 16, 100000, 1), (8, 4, 131072, 1),
+    (32, 12, 1 << 20, 1), (1 << 20, 24, 32, 1), (8, 40, 1 << 20, 1), (3, 3, 70000, 1),
+    (1, 16, 1000, 0), (8, 32, 131072, 0), (8, 64, 1 << 20, 0), (20000, 8, 8, 0),
+    (64, 12, 1 << 20, 1), (64, 12, 262144, 0), (131072, 4, 1000, 1), (100, 12, 1 << 20, 1),
+    (4096, 4, 16384, 0), (131072, 32, 1000, 0), (1024, 784, 1024, 0), (1024, 1024, 100, 0),
+    (2048, 2048, 2048, 0), (2, 2, 2, 0)])
+def test_short_products(rules, M, K, N, short):
+    f = rules.matmul_short_shape
+    f.argtypes = [ctypes.c_longlong] * 3
+    assert f(M, N, K) == short

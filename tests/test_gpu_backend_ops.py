@@ -154,9 +154,13 @@ def test_matmul_matches_oracle_dense(ctx, M, K, N):
     # 32 x 32 tiles: remainders of rows, columns and of the 32-wide K steps
     (33, 1, 31), (1, 31, 97), (32, 32, 32), (95, 67, 65), (31, 36, 513),
     # 64 x 64 tiles (from 160 on), the same remainders
-    (64 * 13 - 63, 33, 64 * 13 - 1), (64 * 10, 64, 64 * 16), (2, 40, 64 * 160)])
+    (64 * 13 - 63, 33, 64 * 13 - 1), (64 * 10, 64, 64 * 16), (2, 40, 64 * 160),
+    # a short K over many tiles: remainders of rows, columns and of its 16-wide
+    # K steps, one side thin either way
+    (1, 1, 64 * 1024), (3, 15, 64 * 1023 + 5), (64 * 1023 + 5, 16, 2), (7, 17, 64 * 1088),
+    (64 * 1984 - 3, 31, 32), (5, 33, 64 * 8192)])
 def test_matmul_tiles_bit_exact(ctx, M, K, N):
-    """Both tile sizes at their edges, row-major and transposed operands,
+    """Each kernel's tiles at their edges, row-major and transposed operands,
     against or_dense (ascending k, separately rounded) bit for bit; the
     entries around the output stay untouched."""
     rng = np.random.default_rng(M + K + N)
