@@ -379,9 +379,10 @@ __device__ __forceinline__ float prob_of(float l, int v, float T,
 // the reference, so the crossing rank can differ where that float sum lies
 // within its rounding error of top_p (a tie).
 // Bound: the passes over the row in registers, one a level on one CU, and the
-// scans between them.  32 rows of 32000 (T 0.8, top-k 50, top-p 0.9): 172 us
-// a call with eight 4-bit levels counted in registers, 45 now; 18 without a
-// filter.
+// scans between them.  32 rows of 32000 (T 0.8, top-k 40, top-p 0.95): 172 us
+// a call with eight 4-bit levels counted in registers, 42 now; 18 without a
+// filter.  Rows of one value 194 / 82 (260 when each of its entries is added to
+// the one bin), 99% masked 171 / 46, few values 194 / 80 to 107.
 // x: p1 of entries v = tid + kThreads i (entries v >= V ignored).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int wave_sum_i(int v) {
@@ -416,20 +417,51 @@ __device__ __forceinline__ void block_filter(const float (&x)[kPer], int V,
       if (use_p) hs[tid + i * kThreads] = 0.0;
     }
     __syncthreads();
+    auto is_cand = [&](int i, uint32_t u) {
+      return tid + i * kThreads < V && (level == 0 || (u >> (shift + bits)) == prefix);
+    };
+    auto count = [&](auto grouped_) {
+      constexpr bool grouped = decltype(grouped_)::value;
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int v = tid + i * kThreads;
-      const uint32_t u = __float_as_uint(x[i]);
-      if (v < V && (level == 0 || (u >> (shift + bits)) == prefix)) {
-        const int d = (int)((u >> shift) & ((1u << bits) - 1u));
-        atomicAdd(&hn[d], 1);
-        if (use_p) {
-          const double q = ((double)x[i] + 1.0) - 1.0;
-          __builtin_amdgcn_ds_atomic_fadd_f64(
-              (__attribute__((address_space(3))) double *)(hs + d), q);
+      for (int i = 0; i < kPer; ++i) {
+        // kept opaque: what is formed from all entries would be formed before
+        // the levels' loop and hold registers through it
+        float xi = x[i];
+        asm volatile("" : "+v"(xi));
+        const uint32_t u = __float_as_uint(xi);
+        const bool cand = is_cand(i, u);
+        auto add = [&](int n) {
+          const int d = (int)((u >> shift) & ((1u << bits) - 1u));
+          atomicAdd(&hn[d], n);
+          if (use_p)
+            __builtin_amdgcn_ds_atomic_fadd_f64(
+                (__attribute__((address_space(3))) double *)(hs + d),
+                (double)n * (((double)xi + 1.0) - 1.0));
+        };
+        if constexpr (grouped) {
+          const uint64_t act = __ballot(cand);
+          if (act == 0) continue;
+          const int first = __builtin_ctzll(act);
+          const uint64_t same =
+              __ballot(cand && u == (uint32_t)__builtin_amdgcn_readlane((int)u, first));
+          if (lane == first) add(__builtin_popcountll(same));
+          else if (cand && !((same >> lane) & 1)) add(1);
+        } else if (cand) {
+          add(1);
         }
       }
-    }
+    };
+    // a wave with many candidates of one value in its first entries (masked or
+    // equal rows, whose additions would wait for each other at one bin) adds
+    // what is equal to the first one of each 64 at once
+    const uint32_t u0 = __float_as_uint(x[0]);
+    const uint64_t act = __ballot(is_cand(0, u0));
+    const int first = act ? __builtin_ctzll(act) : 0;
+    if (__builtin_popcountll(__ballot(
+            is_cand(0, u0) && u0 == (uint32_t)__builtin_amdgcn_readlane((int)u0, first))) >= 8)
+      count(std::true_type{});
+    else
+      count(std::false_type{});
     __syncthreads();
     // the thread's bins from the top: running count and sum before them
     const int top = (1 << bits) - 1 - nb * tid;
