@@ -8,8 +8,12 @@ the row scale, which is an unbounded relative error on entries near zero.
 Where an exact value is cheap (float64), the tests also require the device
 error to be no larger than a small multiple of the oracle's own fp32 error.
 """
+import ctypes
+import functools
 import os
+import subprocess
 import sys
+import tempfile
 
 import numpy as np
 
@@ -46,3 +50,16 @@ def assert_as_accurate(dev, oracle, exact, factor=4.0, what=""):
     bad = e_dev > factor * e_orc + 1e-7 * scale
     assert not bad.any(), (f"{what}: device error {e_dev[bad][:3]} vs oracle "
                            f"{e_orc[bad][:3]}")
+
+
+@functools.lru_cache(None)
+def dispatch_rules():
+    """The library's rules on sizes (csrc/dispatch.hpp), compiled for the host:
+    tests ask them which kernel a shape runs on."""
+    with tempfile.TemporaryDirectory() as d:
+        lib = os.path.join(d, "dispatch_rules.so")
+        subprocess.check_call(
+            ["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC",
+             "-I", os.path.join(ROOT, "neural-network_amd", "csrc"),
+             os.path.join(ROOT, "tests", "cpp", "dispatch_rules.cpp"), "-o", lib])
+        return ctypes.CDLL(lib)

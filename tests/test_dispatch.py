@@ -2,22 +2,15 @@
 the CPU: every shape below was timed with both kernels on an MI355X, and the
 rule takes the faster one (a tie may go either way)."""
 import ctypes
-import os
-import subprocess
 
 import pytest
 
-from gpu_util import ROOT
+from gpu_util import dispatch_rules
 
 
 @pytest.fixture(scope="module")
-def rules(tmp_path_factory):
-    lib = tmp_path_factory.mktemp("dispatch") / "dispatch_rules.so"
-    subprocess.check_call(
-        ["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC",
-         "-I", os.path.join(ROOT, "neural-network_amd", "csrc"),
-         os.path.join(ROOT, "tests", "cpp", "dispatch_rules.cpp"), "-o", str(lib)])
-    return ctypes.CDLL(str(lib))
+def rules():
+    return dispatch_rules()
 
 
 @pytest.mark.parametrize("vs_lds,rows,K,N,tall", [

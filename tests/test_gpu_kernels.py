@@ -10,7 +10,8 @@ import numpy as np
 import pytest
 
 import oracle_py as O
-from gpu_util import assert_as_accurate, assert_rows_close, nnhip, row_rel_err
+from gpu_util import (assert_as_accurate, assert_rows_close, dispatch_rules, nnhip,
+                      row_rel_err)
 
 pytestmark = pytest.mark.gpu
 
@@ -434,7 +435,9 @@ def test_attention_short_launch_query_blocks(ctx, qblk, q8):
 PROMPT_CASES = [(10, 20, 16, 16, 64, 0), (5, 31, 32, 32, 64, 3), (3, 33, 32, 8, 64, 97),
                 (3, 130, 12, 3, 64, 500), (2, 257, 10, 5, 32, 900), (14, 64, 6, 3, 40, 64),
                 (21, 45, 4, 2, 8, 19), (9, 70, 6, 3, 16, 5), (10, 40, 8, 4, 24, 33),
-                (14, 63, 6, 2, 48, 2), (8, 129, 4, 4, 56, 1000)]
+                (14, 63, 6, 2, 48, 2), (8, 129, 4, 4, 56, 1000),
+                # 64 dims over more than 1024 keys: fp32 scores of int8 rows
+                (2, 130, 16, 16, 64, 1000), (3, 100, 16, 4, 64, 1500)]
 
 
 @pytest.mark.parametrize("q8", [False, True])
@@ -449,6 +452,7 @@ def test_attention_prompt(ctx, B, S, H, Hkv, D, past, q8):
     pos0 = rng.integers(0, past + 1, B).astype(np.int32)
     pos0[-1] = past
     cap = int(pos0.max()) + S + 5
+    assert dispatch_rules().attention_prompt_shape(B, S, H, D, q8, cap)
     late = S - 3                       # the new position of the infinite value
     q = rng.standard_normal((B * S, H * D)).astype(np.float32)
     dq, dp = ctx.array(q), ctx.array(pos0)
@@ -917,12 +921,15 @@ def _linear_rows(ctx, x, codes, sc, b, path, step):
     (12 * 128 - 127, 128, 8 * 256),        # 96 tiles, the last with one row
     (4 * 128, 256, 23 * 256 + 64),         # a last column tile of 64
     (1000, 384, 3072), (2050, 512, 1536), (200, 1024, 12288),
-    (8 * 128 + 37, 4096, 12 * 256 - 192)])
+    (8 * 128 + 37, 4096, 12 * 256 - 64),
+    (64, 128, 96 * 256), (70, 512, 128 * 256 - 64)])   # half a row tile
 def test_tall_gemm_matches_short_slices(ctx, rows, K, N):
-    """The 128 x 256-tile GEMM (from 96 tiles on) forms the same exact digit
-    totals and the same rounding as the GEMMs of short inputs, so its rows
-    are bit for bit those of 64-row slices; against float64 within the digit
-    resolution (2^-22 of a row's maximum per entry)."""
+    """The 128 x 256-tile GEMM forms the same exact digit totals and the same
+    rounding as the GEMMs of short inputs, so its rows are bit for bit those of
+    32-row slices; against float64 within the digit resolution (2^-22 of a row's
+    maximum per entry)."""
+    assert dispatch_rules().gemm_tall_shape(rows, K, N, 0)
+    assert not dispatch_rules().gemm_tall_shape(32, K, N, 0)
     rng = np.random.default_rng(rows + K)
     x = rng.standard_normal((rows, K)).astype(np.float32)
     x[::7] *= 1e-3
@@ -931,7 +938,7 @@ def test_tall_gemm_matches_short_slices(ctx, rows, K, N):
     sc = (rng.random(N) * 0.01 + 1e-4).astype(np.float32)
     b = rng.standard_normal(N).astype(np.float32)
     got = _linear_rows(ctx, x, codes, sc, b, 2, rows)
-    np.testing.assert_array_equal(got, _linear_rows(ctx, x, codes, sc, b, 2, 64))
+    np.testing.assert_array_equal(got, _linear_rows(ctx, x, codes, sc, b, 2, 32))
     pick = np.r_[0, 5, 7, rows - 1]
     w = codes.astype(np.float64) * sc[:, None]
     ex = x[pick].astype(np.float64) @ w.T + b
@@ -946,6 +953,7 @@ def test_tall_layernorm_linear(ctx):
     """nnhip_layernorm_linear_w8a32 on a tall input (one LayerNorm launch,
     then the 128 x 256-tile GEMM), with and without ln_out, against float64."""
     rows, K, N = 1570, 512, 2048
+    assert dispatch_rules().gemm_tall_shape(rows, K, N, 1)
     rng = np.random.default_rng(3)
     h = (rng.standard_normal((rows, K)) + 0.2).astype(np.float32)
     g = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
@@ -972,17 +980,28 @@ def test_tall_layernorm_linear(ctx):
     assert np.abs(ys[0] - exy).max() <= 5e-6 * 0.254 * np.sqrt(K) * 6
 
 
-@pytest.mark.parametrize("B,S,q8", [(9, 300, False), (4, 293, False), (9, 300, True)])
-def test_tall_forward_matches_short_batches(ctx, B, S, q8):
-    """A prompt forward whose projections run on the 128 x 256-tile GEMM
-    (bias, residual, SwiGLU and RoPE epilogues, ragged last tiles) gives its
-    first and last sequence the logits and cache rows they get as a batch of
-    two (GEMMs of short inputs): the products are bit-identical, attention
-    and norms are per sequence.  Two sequences of 10 position tiles are what
-    the attention's MFMA kernel starts at, so both sides run it: a sequence
-    alone would run the split-K kernel, whose other rounding (1.4e-7 of a row
-    each, from float64) flips codes of an int8 cache."""
-    d, H, F, V, L = 512, 8, 2048, 640, 2
+@pytest.mark.parametrize("d,B,S,q8,tall", [
+    (512, 9, 300, False, "qkv gu"), (512, 4, 293, False, "gu"), (512, 9, 300, True, "gu"),
+    (1024, 11, 282, False, "qkv o gu down lm"), (1024, 11, 282, True, "o gu down lm")])
+def test_tall_forward_matches_short_batches(ctx, d, B, S, q8, tall):
+    """A prompt forward whose projections run on the 128 x 256-tile GEMM (RoPE,
+    residual, SwiGLU and bias epilogues over ragged last row tiles; `tall` names
+    the products that do) gives its first and last sequence the logits and cache
+    rows they get as a batch of two (GEMMs of short inputs): the products are
+    bit-identical, attention and norms are per sequence.  Two sequences of 9
+    position tiles are enough for the attention's MFMA kernel, so both sides run
+    it: a sequence alone would run the split-K kernel, whose other rounding
+    (1.4e-7 of a row each, from float64) flips codes of an int8 cache."""
+    H, F, V, L = d // 64, 4 * d if d == 512 else 768, 640 if d == 512 else 1056, 2
+    rules, rows = dispatch_rules(), B * S
+    # an int8 append is not in the tall GEMM's epilogue; the down projection's
+    # other kernel is the digit-plane GEMM, the rest's the LDS-resident one
+    shapes = dict(qkv=(d, 3 * d, 1), o=(d, d, 1), gu=(d, 2 * F, 1), down=(F, d, 0), lm=(d, V, 1))
+    assert tall.split() == [n for n, (K, N, lds) in shapes.items() if not (q8 and n == "qkv")
+                            and rules.gemm_tall_shape(rows, K, N, lds)]
+    assert not any(rules.gemm_tall_shape(2 * S, K, N, lds) for K, N, lds in shapes.values())
+    for b in (2, B):
+        assert rules.attention_prompt_shape(b, S, H, 64, q8, S)
     m = nnhip.Decoder(ctx, V, d, H, F, L, 512)
     m.init_normal(5, 0.05)
     m.quantize()
@@ -1021,6 +1040,7 @@ def test_linear_mfma_f32(ctx, rows, K, N, q8):
     the rounding of its sums of float64 (chains of 8 products, two pairwise
     levels, then double and one rounding: 11 roundings at most, each 2^-24 of
     the row's sum of |x w|), and no further from it than the GEMV's rows."""
+    assert dispatch_rules().gemm_f32_shape(rows, N)
     rng = np.random.default_rng(rows * 7 + K)
     x = rng.standard_normal((rows, K)).astype(np.float32)
     b = rng.standard_normal(N).astype(np.float32)
@@ -1063,11 +1083,19 @@ def test_linear_mfma_f32_inf_nan(ctx):
     np.testing.assert_array_equal(y.numpy(), ex.astype(np.float32))
 
 
-@pytest.mark.parametrize("B,S", [(3, 130), (6, 67)])
-def test_unquantised_forward_tall(ctx, B, S):
-    """A prompt forward of an fp32 model, its projections (bias, residual,
-    SwiGLU and RoPE epilogues) on the fp32 MFMA GEMM, against the oracle."""
-    V, d, H, F, L = 300, 192, 6, 300, 2
+@pytest.mark.parametrize("d,H,F,B,S,waves", [
+    # RoPE, residual, SwiGLU, residual of the down projection, bias: the tile of
+    # each (waves over K; 0 the 64 x 64 tiles, -1 the GEMV)
+    (192, 6, 300, 3, 130, (4, -1, 4, -1, 4)), (192, 6, 300, 6, 67, (4, -1, 4, -1, 4)),
+    (256, 8, 300, 3, 130, (4, 4, 4, 4, 4)), (512, 8, 300, 2, 95, (4, 8, 8, 4, -1)),
+    (512, 8, 600, 3, 60, (4, 8, 8, 8, -1)), (512, 8, 300, 3, 50, (8, -1, 8, -1, -1)),
+    (48, 6, 100, 8, 240, (0, 0, 0, 4, 0))])
+def test_unquantised_forward_tall(ctx, d, H, F, B, S, waves):
+    """A prompt forward of an fp32 model, its projections on the fp32 MFMA GEMM
+    with every epilogue over every tile of it, against the oracle."""
+    V, L, rules, rows = 300, 2, dispatch_rules(), B * S
+    assert waves == tuple(rules.gemm_f32_waves(rows, K, N) if rules.gemm_f32_shape(rows, N) else -1
+                          for K, N in ((d, 3 * d), (d, d), (d, 2 * F), (F, d), (d, V)))
     p = O.make_params(V, d, H, F, L, 11, std=0.1)
     m = nnhip.Decoder(ctx, V, d, H, F, L, 256)
     m.set_params(p)
@@ -1076,4 +1104,37 @@ def test_unquantised_forward_tall(ctx, B, S):
     got = m.forward(ids)
     for b in range(B):
         assert_rows_close(got[b], o.forward(ids[b]), what=f"sequence {b}")
+    m.free()
+
+
+@pytest.mark.parametrize("q8", [False, True])
+def test_prompt_after_1024_keys(ctx, q8):
+    """A quantised model's prompt of 150 ids after 900 cached ones: over more
+    than 1024 keys the attention's MFMA kernel is followed by a launch that
+    digitises its rows for the output projection.  An fp32 cache against the
+    oracle, an int8 one against its sequences one by one (split-K kernel and
+    combine)."""
+    V, d, H, F, L, B, past, S = 200, 256, 4, 512, 1, 8, 900, 150
+    rules = dispatch_rules()
+    assert rules.attention_prompt_shape(B, S, H, 64, q8, past + S)
+    assert not rules.attention_prompt_shape(1, S, H, 64, q8, past + S)
+    p = O.make_params(V, d, H, F, L, 5, std=0.1)
+    m = nnhip.Decoder(ctx, V, d, H, F, L, 1100)
+    m.set_params(p)
+    m.quantize()
+    ids = np.random.default_rng(3).integers(0, V, (B, past + S)).astype(np.int32)
+    cache = nnhip.KVCache(m, B, q8)
+    m.forward(ids[:, :past], cache)
+    got = m.forward(ids[:, past:], cache)
+    cache.free()
+    o = None if q8 else O.Model(V, d, H, F, L, 1100, p, True)
+    for b in (0, B - 1):
+        if q8:
+            one = nnhip.KVCache(m, 1, True)
+            m.forward(ids[b:b + 1, :past], one)
+            want = m.forward(ids[b:b + 1, past:], one)[0]
+            one.free()
+        else:
+            want = o.forward(ids[b])[past:]
+        assert_rows_close(got[b], want, what=f"sequence {b}")
     m.free()
