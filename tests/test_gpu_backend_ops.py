@@ -181,11 +181,13 @@ def test_matmul_tiles_bit_exact(ctx, M, K, N):
         assert (got[M] == 7).all() and (got[:, N:] == 7).all()
 
 
-def test_matmul_columns_beyond_one_launch(ctx):
-    """One row times more columns than the threads of one launch cover, every
-    column the same one of b (stride 0): all of them are written, up to the
-    row's end and not past it."""
-    K, N = 33, 2 ** 29 + 70
+@pytest.mark.parametrize("K", [33, 70])   # matmul_short_kernel, matmul_kernel
+def test_matmul_columns_beyond_one_launch(ctx, K):
+    """One row times more columns than the threads of one launch of
+    matmul_kernel cover, every column the same one of b (stride 0): all of them
+    are written, up to the row's end and not past it.  (In one launch only the
+    columns beyond the threads' wrap would be, without an error.)"""
+    N = 2 ** 29 + 70
     a, b = np.arange(1, K + 1, dtype=np.float32), np.full(K, 0.5, np.float32)
     da, db, do = dev(ctx, a), dev(ctx, b), ctx.array(shape=(N + 100,))
     nnhip.call("nnhip_fill_f32", ctx.h, do.p, N + 100, 7.0)
