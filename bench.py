@@ -263,7 +263,8 @@ def verify_step(ctx, t, q8=False):
 # verify forward on 192 rows (d 1024), with the kernel each runs in the
 # library (nnhip_bench_linear path: 1 = GEMV over fp32 rows, 6 = LDS GEMM
 # over digit planes with the lm head's tile statistics, 7 = LDS GEMM over
-# digit planes, 8 = digit-plane GEMM; the digit planes of the output and
+# digit planes or, from 128 rows and enough outputs on, the 128 x 256-tile GEMM
+# (the verify lm head), 8 = digit-plane GEMM; the digit planes of the output and
 # down projections are made by act_quant_kernel, timed apart) and launches
 # per cycle.
 CYCLE_GEMMS = [
@@ -282,7 +283,7 @@ CYCLE_GEMMS = [
     ("verify o", 192, 1024, 1024, 9, "gemm_limb_kernel", 12),
     ("verify gate/up", 192, 1024, 8192, 7, "gemm_lds_kernel", 12),
     ("verify down", 192, 4096, 1024, 8, "gemm_limb_kernel", 12),
-    ("verify lm head", 192, 1024, 32000, 6, "gemm_lds_kernel", 1),
+    ("verify lm head", 192, 1024, 32000, 7, "gemm_tall_kernel", 1),
 ]
 
 

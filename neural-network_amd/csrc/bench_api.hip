@@ -145,7 +145,7 @@ int nnhip_bench_spec_accept(nnhip_ctx *ctx, int B, int k, int V, float T,
 // included), 5 = LDS GEMM with LayerNorm (gamma 1, beta 0) in its prologue,
 // 6 = LDS GEMM over digit planes made once, with tile statistics; over
 // digit planes made once, the GEMM alone: 7 = LDS GEMM, 8 = digit-plane
-// GEMM.
+// GEMM; 4, 7, 8 (and 2) run tall shapes on the 128 x 256-tile GEMM.
 int nnhip_bench_linear(nnhip_ctx *ctx, int rows, int K, int N, int path,
                        int iters, int nbuf, float *ms) {
   return guard([&] {
