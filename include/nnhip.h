@@ -254,11 +254,14 @@ int nnhip_quantize_w8(nnhip_ctx *ctx, const float *w, int in, int out,
 int nnhip_quantize_w4(nnhip_ctx *ctx, const float *w, int in, int out,
                       int8_t *codes, float *scales);
 /* QuantizedDense::forward (quantization.cpp:127-147): y [rows][N] =
- * x [rows][K] . (codes * scales)^T + bias.  path: 0 auto, 1 fp32 GEMV,
+ * x [rows][K] . (codes * scales)^T + bias.  path: 0 auto, 1 fp32 products
+ * (the GEMV, from 16 rows and 90000 outputs on the fp32 MFMA GEMM: another
+ * summation order, so a row's last bits depend on how many rows a call has),
  * 2 int8-digit MFMA GEMM (K % 128 == 0, N % 64 == 0), 3 MFMA GEMM with the
  * digits formed in LDS from x, 4 the same GEMM fed with digit planes
- * (3 and 4: K in {128, 256, 512, 1024}, N % 32 == 0).  The MFMA paths (2-4)
- * agree bit for bit.  Stream-ordered: the digit planes and the codes in the
+ * (3 and 4: K in {128, 256, 512, 1024}, N % 32 == 0).  Paths 2 and 4 run tall
+ * inputs on a GEMM of 128 x 256 tiles.  The digit paths (2-4) agree bit for
+ * bit.  Stream-ordered: the digit planes and the codes in the
  * MFMA operand layout go to scratch the context keeps and reuses, which
  * grows (after draining the stream) only when a call needs more. */
 int nnhip_linear_w8a32(nnhip_ctx *ctx, const float *x, int rows, int K,
@@ -271,8 +274,11 @@ int nnhip_linear_w8a32(nnhip_ctx *ctx, const float *x, int rows, int K,
  * and LN(h) into ln_out when it is not NULL.  K in {128, 256, 512, 1024},
  * N % 32 == 0.  Rows below 16 run on the GEMV with the LayerNorm as its
  * prologue (the decode path of short batches), others on the LDS-resident
- * MFMA GEMM with the LayerNorm in its prologue.  Stream-ordered, with the
- * context's scratch as nnhip_linear_w8a32. */
+ * MFMA GEMM with the LayerNorm in its prologue; tall inputs (from 128 rows and
+ * 3.1 M outputs on, pointers aligned to 16 bytes) get a LayerNorm launch that
+ * writes digit planes for the GEMM of 128 x 256 tiles.  Stream-ordered, with the
+ * context's scratch as nnhip_linear_w8a32: N*K bytes for the codes and, for
+ * tall inputs, 3*K bytes a row. */
 int nnhip_layernorm_linear_w8a32(nnhip_ctx *ctx, const float *h, int rows,
                                  int K, const float *gamma, const float *beta,
                                  float *ln_out, const int8_t *codes,
@@ -295,7 +301,8 @@ int nnhip_linear_w8a32_noalloc(nnhip_ctx *ctx, const float *x, int rows,
                                int K, const int8_t *codes,
                                const float *scales, const float *bias, int N,
                                float *y, int path);
-/* Dense::forward (layer.cpp:162-171) with w [N][K] fp32 (transposed). */
+/* Dense::forward (layer.cpp:162-171) with w [N][K] fp32 (transposed): the GEMV,
+ * from 16 rows and 90000 outputs on the fp32 MFMA GEMM (path 1 above). */
 int nnhip_linear_f32(nnhip_ctx *ctx, const float *x, int rows, int K,
                      const float *w, const float *bias, int N, float *y);
 /* The MFMA path's exact integers: row exponents rexp [rows], digits
@@ -322,7 +329,9 @@ int nnhip_rope_kv_append_gqa(nnhip_ctx *ctx, const float *qkv, int B, int S,
 /* Fused causal attention of MultiHeadAttention::forward (layer.cpp:842-952)
  * for S queries per sequence: q [B*S][H*D], kcache / vcache [B][Hkv][cap][D]
  * holding pos0[b] + S valid entries; query s sees keys j <= pos0[b] + s.
- * out [B*S][H*D]. */
+ * out [B*S][H*D].  The kernel is chosen by the launch's sizes (prompts in tiles
+ * of 32 queries on the MFMA, others split over the keys), so a sequence's last
+ * bits depend on the batch it is in. */
 int nnhip_attention_kq(nnhip_ctx *ctx, const float *q, const float *kcache,
                        const float *vcache, int cap, const int32_t *pos0,
                        int B, int S, int H, int Hkv, int D, float *out);
@@ -471,7 +480,8 @@ int nnhip_bench_spec_accept(nnhip_ctx *ctx, int B, int k, int V,
  * digit split included), 5 = LDS GEMM with LayerNorm in its prologue,
  * 6 = LDS GEMM over digit planes made once, with the lm head's tile
  * softmax statistics (K of 512 or 1024); the GEMM alone over digit planes
- * made once: 7 = LDS GEMM, 8 = digit-plane GEMM, 9 = digit-plane GEMM with
+ * made once: 7 = LDS GEMM (tall shapes: the GEMM of 128 x 256 tiles, as for 4
+ * and 8), 8 = digit-plane GEMM, 9 = digit-plane GEMM with
  * one exponent per 64-wide K chunk (the output projection's; K <= 2048). */
 int nnhip_bench_linear(nnhip_ctx *ctx, int rows, int K, int N, int path,
                        int iters, int nbuf, float *ms);

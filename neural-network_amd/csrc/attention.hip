@@ -759,9 +759,10 @@ __global__ __launch_bounds__(kWave * W, W == 4 ? 2 : 1) void attn_kernel(
 //    wave reads one row; with more than 32 dims, dims 2 c and 2 c + 1 go to
 //    two accumulators).
 // Precision: score sums are 8-product fp32 chains added pairwise; a chunk's
-// 32 products of PV are chained from zero and added to the running rows.
-// int8 rows of 64 dims take the exact integer scores of attn_kernel's MS
-// path; other int8 rows become (float)code * scale as there.
+// 32 products of PV are four chains of 8 added pairwise, then added to the
+// running rows.  int8 rows of 64 dims in caches of up to 1024 keys take the
+// exact integer scores of attn_kernel's MS path; other int8 rows become
+// (float)code * scale, as there.
 // A key after some of the tile's queries has p = 0 for them; a V row of such
 // a chunk that is not finite would still spoil their sums (0 * inf), so a
 // chunk with one is summed key by key over the queries that see it.

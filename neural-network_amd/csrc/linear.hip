@@ -1126,9 +1126,9 @@ __global__ __launch_bounds__(kLdsThreads) void gemm_lds_kernel(
 // LDS reads; the exact int32 sums of each digit plane stay in registers for
 // the whole of K (|sum| < 4096 * 127 * 128 < 2^31 at the largest K), so the
 // totals are those of the other two GEMMs and the outputs bit-identical.
-// Bound: the MFMAs.  A stage is 1776 MFMA cycles a SIMD; it takes 0.9 us with
-// few tiles running and 1.3 us with all CUs busy (the rate a large bf16
-// product reaches on this card, 45% of its peak).  8192 x 8192 at K = 1024:
+// Bound: the MFMAs.  A stage is 48 MFMAs of 32 cycles a SIMD, 0.64 us at 2.4
+// GHz; it takes 0.9 us with few tiles running and 1.3 us with all CUs busy (the
+// rate a large bf16 product reaches on this card, 45% of its peak).  8192 x 8192 at K = 1024:
 // 220 us, 1.9 POP/s of digit products (gemm_lds_kernel 333, gemm_limb_kernel
 // 752); 8192 x 1024 at K = 4096: 90 us, 2.3 POP/s (249).  128 x 256 and not
 // 256 x 128: the digits are three bytes an entry and the codes one, so the

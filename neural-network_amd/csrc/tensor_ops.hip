@@ -122,15 +122,17 @@ __global__ __launch_bounds__(kBlock) void unary_kernel(
 // thread; K goes through LDS 32 at a time, the next 32 held in registers
 // meanwhile (two LDS buffers, one barrier per 32).  Every output adds its
 // products in ascending k, each product and sum rounded on its own: 2 VALU
-// instructions a product, so 39 TFLOP/s (at 2.4 GHz) is the card's bound and
-// no split of K is possible.  A wave alone on its SIMD issues one instruction
-// in 8 cycles, so tiles are spread over 8 waves, and the operands are kept
-// with k innermost, so that one 16-byte LDS read serves four k's (rows of 36
-// words: the 16 columns a wave reads fall on different banks).  Operand loads
-// run along whichever dimension of the view is the denser one, so a
-// transposed view reads as coalesced as a row-major one.
+// instructions a product, and no split of K is possible.  A loop of nothing
+// but such multiplications and additions on vector registers reaches 34
+// TFLOP/s with one wave a SIMD (4.6 cycles an instruction at 2.4 GHz), 64 with
+// two and 75 with sixteen (2.1 cycles), so tiles are spread over 8 waves, two a
+// SIMD.  The operands are kept with k innermost, so that one 16-byte LDS read
+// serves four k's (rows of 36 words: the 16 columns a wave reads fall on
+// different banks).  Operand loads run along whichever dimension of the view
+// is the denser one, so a transposed view reads as coalesced as a row-major
+// one.
 // 1024 x 784 x 1024: 134 -> 51 us, 1024 x 1024 x 100: 165 -> 27, 2048 x 2048
-// x 2048: 480 -> 385 (44.7 TFLOP/s).
+// x 2048: 487 -> 393 (43.8 TFLOP/s, 58% of that loop's rate).
 constexpr int kKT = 32;
 // 64 x 64 tiles from 160 of them on, below it 32 x 32 ones (four times the
 // workgroups): 192 tiles 32.2 / 34.3 us (64 / 32), 128 tiles 30.8 / 23.8, 32
